@@ -98,23 +98,23 @@ struct Arena {
   // [3][slots] of the stage buffers, node extrema [slots*NCL][2] (the
   // limited components: all NC in 3D, component 0 in 2D)
   DevBuf<double> lmean, ltheta, lext;
-  DevBuf<double> invJ, inv_vol, jgeo, iprm, idt, ipost;
+  DevBuf<double> invJ, inv_vol, geom, iprm, idt, ipost;  // geom: one table per instance slot
   DevBuf<int> conn;  // limiter: partner slot per face
-  DevBuf<int4> jobs;
+  DevBuf<int2> jobs;
   DevBuf<unsigned short> ipr;
-  DevBuf<int> tile_count, tile_inst, iactive, isteps, insteps, ifail;
+  DevBuf<int> tile_count, tile_type, tile_inst, iactive, isteps, insteps, ifail;
   void swap(Arena &o) noexcept {
     for (int k = 0; k < 3; ++k) qd[k].swap(o.qd[k]), qf[k].swap(o.qf[k]);
-    lmean.swap(o.lmean), ltheta.swap(o.ltheta), lext.swap(o.lext), invJ.swap(o.invJ), inv_vol.swap(o.inv_vol), jgeo.swap(o.jgeo), iprm.swap(o.iprm);
+    lmean.swap(o.lmean), ltheta.swap(o.ltheta), lext.swap(o.lext), invJ.swap(o.invJ), inv_vol.swap(o.inv_vol), geom.swap(o.geom), iprm.swap(o.iprm);
     idt.swap(o.idt), ipost.swap(o.ipost), conn.swap(o.conn), jobs.swap(o.jobs), ipr.swap(o.ipr);
-    tile_count.swap(o.tile_count), tile_inst.swap(o.tile_inst), iactive.swap(o.iactive), isteps.swap(o.isteps);
+    tile_count.swap(o.tile_count), tile_type.swap(o.tile_type), tile_inst.swap(o.tile_inst), iactive.swap(o.iactive), isteps.swap(o.isteps);
     insteps.swap(o.insteps), ifail.swap(o.ifail);
   }
   size_t bytes() const {
     size_t b = 0;
     for (int k = 0; k < 3; ++k) b += qd[k].bytes() + qf[k].bytes();
-    return b + lmean.bytes() + ltheta.bytes() + lext.bytes() + invJ.bytes() + inv_vol.bytes() + jgeo.bytes() + iprm.bytes() + idt.bytes() +
-           ipost.bytes() + conn.bytes() + jobs.bytes() + ipr.bytes() + tile_count.bytes() + tile_inst.bytes() +
+    return b + lmean.bytes() + ltheta.bytes() + lext.bytes() + invJ.bytes() + inv_vol.bytes() + geom.bytes() + iprm.bytes() + idt.bytes() +
+           ipost.bytes() + conn.bytes() + jobs.bytes() + ipr.bytes() + tile_count.bytes() + tile_type.bytes() + tile_inst.bytes() +
            iactive.bytes() + isteps.bytes() + insteps.bytes() + ifail.bytes();
   }
 };
@@ -241,9 +241,9 @@ size_t instance_bytes(const ElemTables &t, int NP, int NC, int NFP, int dim, int
   size_t b = 3 * slots * NP * NC * word;                            // state trio
   b += slots * (dim * dim + 1) * sizeof(double);                    // invJ, inv_vol
   b += slots * (dim + 1) * sizeof(int);                             // limiter neighbours
-  b += js * (sizeof(int4) + 4 * sizeof(double) + NFP * sizeof(unsigned short));  // jobs, geometry, partner nodes
-  b += tiles * 2 * sizeof(int);                                     // tile_count, tile_inst
-  b += (MXM_PRM_MAX + 2) * sizeof(double) + 4 * sizeof(int);        // per-instance scalars
+  b += js * (sizeof(int2) + NFP * sizeof(unsigned short));          // jobs, partner nodes
+  b += tiles * 3 * sizeof(int);                                     // tile_count, tile_type, tile_inst
+  b += (MXM_PRM_MAX + 2 + t.geom.size()) * sizeof(double) + 4 * sizeof(int);  // per-instance scalars, geometry
   if (limiter) b += slots * (3 * NC + 2 * (dim == 3 ? NC : 1) + 3) * sizeof(double);  // means, factors, extrema
   return b;
 }
@@ -253,9 +253,9 @@ size_t instance_bytes(const ElemTables &t, int NP, int NC, int NFP, int dim, int
 struct InstImage {
   std::vector<double> ij, iv, geo, prm;
   std::vector<int> cn;
-  std::vector<int4> jb;
+  std::vector<int2> jb;
   std::vector<unsigned short> pr;
-  std::vector<int> tc, ti;
+  std::vector<int> tc, ty, ti;
   double dt = 0.0, post = 1.0;
   int active = 0, steps = 0, nsteps = 0;
 };
@@ -271,7 +271,8 @@ InstImage inst_image(const BGroup &g, const BInst &in, int bt, int sl, int maxj)
   m.cn.resize(slots * NF);
   for (size_t s = 0; s < slots * NF; ++s) m.cn[s] = t.conn[s] + bs;
   m.jb.resize((size_t)lt * maxj);
-  m.geo.assign((size_t)lt * maxj * 4, 0.0);
+  m.geo = t.geom;
+  m.ty = t.tile_type;
   m.pr.assign((size_t)lt * maxj * NFP, 0);
   m.tc.resize(lt);
   m.ti.assign(lt, sl);
@@ -281,11 +282,10 @@ InstImage inst_image(const BGroup &g, const BInst &in, int bt, int sl, int maxj)
       const size_t dj = (size_t)T * maxj + j;
       if (j < lmj) {
         const size_t sj = (size_t)T * lmj + j;
-        m.jb[dj] = int4{t.fj.jobs[sj * 4], t.fj.jobs[sj * 4 + 1] + bs, t.fj.jobs[sj * 4 + 2], t.fj.jobs[sj * 4 + 3]};
-        for (int c = 0; c < 4; ++c) m.geo[dj * 4 + c] = t.fj.geo[sj * 4 + c];
+        m.jb[dj] = int2{t.fj.jobs[sj * 2], t.fj.jobs[sj * 2 + 1] + bs};
         for (int r = 0; r < NFP; ++r) m.pr[dj * NFP + r] = t.fj.ipr[sj * NFP + r];
       } else {
-        m.jb[dj] = int4{-1, (bt + T) * epb, 0, 0};  // padding job: in-bounds partner, skipped
+        m.jb[dj] = int2{-1, (bt + T) * epb};  // padding job: in-bounds partner, skipped
       }
     }
   }
@@ -513,10 +513,11 @@ struct Batch {
         {g.ar.invJ.p + bs * dd, m.ij.data(), m.ij.size() * sizeof(double)},
         {g.ar.inv_vol.p + bs, m.iv.data(), m.iv.size() * sizeof(double)},
         {g.ar.conn.p + bs * NF, m.cn.data(), m.cn.size() * sizeof(int)},
-        {g.ar.jobs.p + (size_t)bt * g.maxj, m.jb.data(), m.jb.size() * sizeof(int4)},
-        {g.ar.jgeo.p + (size_t)bt * g.maxj * 4, m.geo.data(), m.geo.size() * sizeof(double)},
+        {g.ar.jobs.p + (size_t)bt * g.maxj, m.jb.data(), m.jb.size() * sizeof(int2)},
+        {g.ar.geom.p + (size_t)sl * m.geo.size(), m.geo.data(), m.geo.size() * sizeof(double)},
         {g.ar.ipr.p + (size_t)bt * g.maxj * g.NFP, m.pr.data(), m.pr.size() * sizeof(unsigned short)},
         {g.ar.tile_count.p + bt, m.tc.data(), m.tc.size() * sizeof(int)},
+        {g.ar.tile_type.p + bt, m.ty.data(), m.ty.size() * sizeof(int)},
         {g.ar.tile_inst.p + bt, m.ti.data(), m.ti.size() * sizeof(int)},
         {g.ar.iprm.p + (size_t)sl * MXM_PRM_MAX, m.prm.data(), MXM_PRM_MAX * sizeof(double)},
         {g.ar.idt.p + sl, &m.dt, sizeof(double)},
@@ -648,17 +649,19 @@ struct Batch {
       state_trio(na.qd, g.ar.qd);
     else
       state_trio(na.qf, g.ar.qf);
-    std::vector<double> ij(slots * dd, 0.0), iv(slots, 0.0), geo((size_t)cap_tiles * maxj * 4, 0.0);
+    std::vector<double> ij(slots * dd, 0.0), iv(slots, 0.0);
+    const size_t gl = stage_geom_len(g.dim);
+    std::vector<double> geo(cap_slots * gl, 0.0);
     std::vector<int> cn(slots * NF);
-    std::vector<int4> jb((size_t)cap_tiles * maxj);
+    std::vector<int2> jb((size_t)cap_tiles * maxj);
     std::vector<unsigned short> pr((size_t)cap_tiles * maxj * NFP, 0);
-    std::vector<int> tc(cap_tiles, 0), ti(cap_tiles, 0);
+    std::vector<int> tc(cap_tiles, 0), ty(cap_tiles, 0), ti(cap_tiles, 0);
     std::vector<double> iprm((size_t)cap_slots * MXM_PRM_MAX, 0.0), idt(cap_slots, 0.0), ipost(cap_slots, 1.0);
     std::vector<int> iact(cap_slots, 0), ist(cap_slots, 0), inst_n(cap_slots, 0), ifl(cap_slots, 0);
     for (int s = 0; s < (int)slots; ++s)
       for (int lf = 0; lf < NF; ++lf) cn[(size_t)s * NF + lf] = s;
     for (int T = 0; T < cap_tiles; ++T)
-      for (int j = 0; j < maxj; ++j) jb[(size_t)T * maxj + j] = int4{-1, T * epb, 0, 0};
+      for (int j = 0; j < maxj; ++j) jb[(size_t)T * maxj + j] = int2{-1, T * epb};
     std::vector<int> new_base(ni);
     int bt = 0;
     for (int k = 0; k < ni; ++k) {
@@ -670,9 +673,10 @@ struct Batch {
       std::copy(m.iv.begin(), m.iv.end(), iv.begin() + bs);
       std::copy(m.cn.begin(), m.cn.end(), cn.begin() + bs * NF);
       std::copy(m.jb.begin(), m.jb.end(), jb.begin() + (size_t)bt * maxj);
-      std::copy(m.geo.begin(), m.geo.end(), geo.begin() + (size_t)bt * maxj * 4);
+      std::copy(m.geo.begin(), m.geo.end(), geo.begin() + (size_t)sl * gl);
       std::copy(m.pr.begin(), m.pr.end(), pr.begin() + (size_t)bt * maxj * NFP);
       std::copy(m.tc.begin(), m.tc.end(), tc.begin() + bt);
+      std::copy(m.ty.begin(), m.ty.end(), ty.begin() + bt);
       std::copy(m.ti.begin(), m.ti.end(), ti.begin() + bt);
       std::copy(m.prm.begin(), m.prm.end(), iprm.begin() + (size_t)sl * MXM_PRM_MAX);
       idt[sl] = m.dt, ipost[sl] = m.post, iact[sl] = m.active, ist[sl] = m.steps, inst_n[sl] = m.nsteps;
@@ -683,9 +687,10 @@ struct Batch {
     na.inv_vol.upload(iv.data(), iv.size());
     na.conn.upload(cn.data(), cn.size());
     na.jobs.upload(jb.data(), jb.size());
-    na.jgeo.upload(geo.data(), geo.size());
+    na.geom.upload(geo.data(), geo.size());
     na.ipr.upload(pr.data(), pr.size());
     na.tile_count.upload(tc.data(), tc.size());
+    na.tile_type.upload(ty.data(), ty.size());
     na.tile_inst.upload(ti.data(), ti.size());
     na.iprm.upload(iprm.data(), iprm.size());
     na.idt.upload(idt.data(), idt.size());
@@ -794,10 +799,10 @@ struct Batch {
     a.dt = 0.0, a.post_scale = 1.0;
     // GLM decay per instance (factor 1 where alpha_d = 0)
     a.post_comp = s == 2 && g.phys == MXM_PHYS_MHDGLM2D ? 6 : -1;
-    a.tile_count = ar.tile_count.p;
-    a.invJ = ar.invJ.p, a.inv_vol = ar.inv_vol.p;
+    a.tile_count = ar.tile_count.p, a.tile_type = ar.tile_type.p;
+    a.geom = ar.geom.p;
     a.Dt = g.Dt.p, a.Lt = g.Lt.p, a.Aop = g.Aop.p, a.fmap = g.fmap.p;
-    a.jobs = ar.jobs.p, a.jgeo = ar.jgeo.p, a.ipr = ar.ipr.p, a.maxj = g.maxj, a.ntiles = g.grid_tiles;
+    a.jobs = ar.jobs.p, a.ipr = ar.ipr.p, a.maxj = g.maxj, a.ntiles = g.grid_tiles;
     return a;
   }
 

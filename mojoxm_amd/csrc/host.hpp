@@ -77,24 +77,30 @@ struct Tiling {
 };
 Tiling build_tiling(const HostMesh &m, int epb, int NFP);
 
+// Distinct face geometries of a lattice mesh, at most: 12 periodic face
+// types and 6 one-sided boundary ones in 3D, 3 and 2 in 2D.
+constexpr int max_face_geo(int dim) { return dim == 3 ? 18 : 5; }
+// Elements of a lattice cell
+constexpr int cell_elems(int dim) { return dim == 3 ? 6 : 2; }
+
 // Face-flux work lists of the stage kernel.  Within a tile, a face whose
 // two sides both lie in the tile is evaluated once (by its side-0
 // element), which also writes the negated flux into the partner's slots.
-// Every tile owns `maxj` job slots (padding: packed = -1), so the records a
-// thread needs are addressed from the tile index alone:
-//   jobs[T*maxj + j]  el | lf << 7 | (partner_local + 1 or 0) << 9 |
-//                     partner_lf << 16 | pslot << 18, the partner's device
-//                     slot, the face id, the connectivity flags
-//   geo[(T*maxj + j)*4 + 0..3]  face normal (x, y, z; 0 beyond ND), area
+// Every tile owns `maxj` job slots (padding: the record is -1), so the
+// records a thread needs are addressed from the tile index alone:
+//   jobs[(T*maxj + j)*2]      el | lf << 7 | (partner_local + 1 or 0) << 9 |
+//                     partner_lf << 16 | side << 18 | bc << 19 |
+//                     geometry << 22 (an entry of geo)
+//   jobs[(T*maxj + j)*2 + 1]  the partner's device slot
 //   ipr[(T*maxj + j)*NFP + r]   partner node meeting slot r | (partner's
 //                     reference slot for the paired write) << 8
-// pslot_tab[pslot*NFP + r] is the partner's reference slot meeting slot r.
+// geo[4*g + 0..3]     the mesh's distinct face normals (x, y, z; 0 beyond
+//                     ND) with their areas, max_face_geo entries
 struct FaceJobs {
   int maxj = 0;
-  std::vector<int32_t> jobs, pslot_tab;
+  std::vector<int32_t> jobs;
   std::vector<double> geo;
   std::vector<uint16_t> ipr;
-  int npslot = 0;
 };
 FaceJobs build_face_jobs(const HostMesh &m, const RefElem &re, const Connectivity &c, const Tiling &t);
 

@@ -550,9 +550,21 @@ FaceJobs build_face_jobs(const HostMesh &m, const RefElem &re, const Connectivit
   const int NF = m.NF, NFP = m.NFP, epb = t.epb, ND = m.dim;
   if (m.NP > 255 || NFP > 255) throw std::runtime_error("jobs: node index does not fit 8 bits");
   FaceJobs J;
-  std::vector<std::vector<int>> pats;
   std::vector<int> pat(NFP);
-  // per tile: job records (4 ints) and the partner node of each slot
+  // the distinct face geometries, in order of first use
+  const int max_geo = max_face_geo(ND);
+  J.geo.assign((size_t)max_geo * 4, 0.0);
+  int ngeo = 0;
+  auto geometry = [&](int fid) {
+    double v[4] = {0.0, 0.0, 0.0, m.face_area[fid]};
+    for (int d = 0; d < ND; ++d) v[d] = m.face_normal[(size_t)fid * ND + d];
+    for (int g = 0; g < ngeo; ++g)
+      if (std::equal(v, v + 4, &J.geo[(size_t)g * 4])) return g;
+    if (ngeo == max_geo) throw std::runtime_error("jobs: more face geometries than a lattice has");
+    std::copy(v, v + 4, &J.geo[(size_t)ngeo * 4]);
+    return ngeo++;
+  };
+  // per tile: job records (2 ints) and the partner node of each slot
   std::vector<std::vector<int32_t>> tj(t.ntiles);
   std::vector<std::vector<int32_t>> tn(t.ntiles);
   for (int T = 0; T < t.ntiles; ++T) {
@@ -575,7 +587,7 @@ FaceJobs build_face_jobs(const HostMesh &m, const RefElem &re, const Connectivit
               plf = q;
         const bool pair = plf >= 0;
         if (pair && side == 1) continue;  // evaluated by the side-0 element
-        int packed = el | (lf << 7);
+        int packed = el | (lf << 7) | (side << 18) | (bc << 19) | (geometry(fid) << 22);
         for (int r = 0; r < NFP; ++r) pat[r] = 0;
         if (pair) {
           for (int r = 0; r < NFP; ++r) {
@@ -586,33 +598,24 @@ FaceJobs build_face_jobs(const HostMesh &m, const RefElem &re, const Connectivit
             if (rs < 0) throw std::runtime_error("jobs: partner slot not found");
             pat[r] = rs;
           }
-          int id = -1;
-          for (size_t p = 0; p < pats.size(); ++p)
-            if (pats[p] == pat) id = (int)p;
-          if (id < 0) {
-            id = (int)pats.size();
-            pats.push_back(pat);
-          }
-          if (id >= (1 << 13)) throw std::runtime_error("jobs: too many slot patterns");
-          packed |= ((pl + 1) << 9) | (plf << 16) | (id << 18);
+          packed |= ((pl + 1) << 9) | (plf << 16);
         }
-        tj[T].insert(tj[T].end(), {packed, pdev, fid, cn[2]});
+        tj[T].insert(tj[T].end(), {packed, pdev});
         for (int r = 0; r < NFP; ++r) tn[T].push_back(c.perm_tab[(size_t)pid * NFP + r] | (pat[r] << 8));
       }
-    J.maxj = std::max(J.maxj, (int)(tj[T].size() / 4));
+    J.maxj = std::max(J.maxj, (int)(tj[T].size() / 2));
   }
-  J.npslot = (int)pats.size();
   // Every (element, face, slot) of a tile must be written exactly once.
   std::vector<int> hits((size_t)epb * NF * NFP);
   for (int T = 0; T < t.ntiles; ++T) {
     const int nE = t.count[T];
     std::fill(hits.begin(), hits.end(), 0);
-    for (size_t j = 0; j < tj[T].size() / 4; ++j) {
-      const int job = tj[T][j * 4], el = job & 127, lf = (job >> 7) & 3, pin = (job >> 9) & 127;
+    for (size_t j = 0; j < tj[T].size() / 2; ++j) {
+      const int job = tj[T][j * 2], el = job & 127, lf = (job >> 7) & 3, pin = (job >> 9) & 127;
       if (el >= nE || (pin && pin - 1 >= nE)) throw std::runtime_error("jobs: element outside its tile");
       for (int r = 0; r < NFP; ++r) {
         ++hits[((size_t)el * NF + lf) * NFP + r];
-        if (pin) ++hits[((size_t)(pin - 1) * NF + ((job >> 16) & 3)) * NFP + pats[job >> 18][r]];
+        if (pin) ++hits[((size_t)(pin - 1) * NF + ((job >> 16) & 3)) * NFP + (tn[T][j * NFP + r] >> 8)];
       }
     }
     for (int k = 0; k < nE * NF * NFP; ++k)
@@ -620,27 +623,21 @@ FaceJobs build_face_jobs(const HostMesh &m, const RefElem &re, const Connectivit
   }
   // fixed-stride device tables
   const size_t slots = (size_t)t.ntiles * J.maxj;
-  J.jobs.assign(slots * 4, 0);
-  J.geo.assign(slots * 4, 0.0);
+  J.jobs.assign(slots * 2, 0);
   J.ipr.assign(slots * NFP, 0);
   for (int T = 0; T < t.ntiles; ++T) {
-    const size_t nj = tj[T].size() / 4;
+    const size_t nj = tj[T].size() / 2;
     for (size_t j = 0; j < (size_t)J.maxj; ++j) {
       const size_t s = (size_t)T * J.maxj + j;
       if (j >= nj) {
-        J.jobs[s * 4 + 0] = -1;
-        J.jobs[s * 4 + 1] = T * epb;
+        J.jobs[s * 2 + 0] = -1;
+        J.jobs[s * 2 + 1] = T * epb;
         continue;
       }
-      for (int k = 0; k < 4; ++k) J.jobs[s * 4 + k] = tj[T][j * 4 + k];
-      const int fid = tj[T][j * 4 + 2];
-      for (int d = 0; d < ND; ++d) J.geo[s * 4 + d] = m.face_normal[(size_t)fid * ND + d];
-      J.geo[s * 4 + 3] = m.face_area[fid];
+      for (int k = 0; k < 2; ++k) J.jobs[s * 2 + k] = tj[T][j * 2 + k];
       for (int r = 0; r < NFP; ++r) J.ipr[s * NFP + r] = (uint16_t)tn[T][j * NFP + r];
     }
   }
-  for (auto &p : pats) J.pslot_tab.insert(J.pslot_tab.end(), p.begin(), p.end());
-  if (J.pslot_tab.empty()) J.pslot_tab.assign(NFP, 0);
   return J;
 }
 

@@ -203,6 +203,10 @@ struct ElemTables {
   FaceJobs fj;
   std::vector<double> invJ, inv_vol;
   std::vector<int> conn;  // limiter neighbours: the partner slot of each face (its own slot on a boundary)
+  // the stage kernel's geometry (StageArgs::geom): the distinct face normals
+  // and areas, then invJ and inv_vol of each element of a lattice cell
+  std::vector<double> geom;
+  std::vector<int> tile_type;  // cell element of each tile's first slot
 };
 
 // wide: tiles of the wide tile size (stage_epb)
@@ -227,6 +231,23 @@ inline ElemTables build_elem_tables(const HostMesh &m, const RefElem &re, int nc
     t.inv_vol[sl] = m.elem_inv_vol[e];
   }
   t.fj = build_face_jobs(m, re, cn, t.til);
+  t.geom = std::move(t.fj.geo);
+  const int epc = cell_elems(m.dim);
+  for (int y = 0; y < epc; ++y) {
+    t.geom.insert(t.geom.end(), &m.elem_invJ[(size_t)y * dd], &m.elem_invJ[(size_t)y * dd] + dd);
+    t.geom.push_back(m.elem_inv_vol[y]);
+  }
+  // every element has the geometry of its place in its cell, and a tile's
+  // slots run through those places in order
+  t.tile_type.assign(t.til.ntiles, 0);
+  for (int sl = 0; sl < Kd; ++sl) {
+    const int e = t.til.ref_of[sl], T = sl / t.til.epb, el = sl - T * t.til.epb;
+    if (e < 0) continue;
+    if (el == 0) t.tile_type[T] = e % epc;
+    if ((t.tile_type[T] + el) % epc != e % epc || m.elem_inv_vol[e] != m.elem_inv_vol[e % epc] ||
+        std::memcmp(&m.elem_invJ[(size_t)e * dd], &m.elem_invJ[(size_t)(e % epc) * dd], dd * sizeof(double)))
+      throw std::runtime_error("tables: an element without the geometry of its place in its cell");
+  }
   return t;
 }
 

@@ -62,12 +62,12 @@ struct Solver {
   // buffers (q, q1, q2), node extrema [Kd*NCL][2] of the last stage output
   // (the limited components: all NC in 3D, component 0 in 2D)
   DevBuf<double> lmean, ltheta, lext;
-  DevBuf<double> invJ, inv_vol, jgeo, Dt, Lt, w, dprm;
+  DevBuf<double> invJ, inv_vol, geom, Dt, Lt, w, dprm;
   DevBuf<double> Dn, dpart, dout;  // diagnostics: nodal derivative, tile partials, results
   DevBuf<float> Aop;
   DevBuf<int> conn;  // limiter: partner slot per face
-  DevBuf<int> fmap, tile_count;
-  DevBuf<int4> jobs;
+  DevBuf<int> fmap, tile_count, tile_type;
+  DevBuf<int2> jobs;
   DevBuf<unsigned short> ipr;
   int maxj = 0;
   // Device element order: tiles of lattice cells, each contiguous
@@ -174,8 +174,9 @@ struct Solver {
     conn.upload(t.conn.data(), t.conn.size());
     maxj = t.fj.maxj;
     tile_count.upload(til.count.data(), til.count.size());
-    jobs.upload(reinterpret_cast<const int4 *>(t.fj.jobs.data()), t.fj.jobs.size() / 4);
-    jgeo.upload(t.fj.geo.data(), t.fj.geo.size());
+    tile_type.upload(t.tile_type.data(), t.tile_type.size());
+    jobs.upload(reinterpret_cast<const int2 *>(t.fj.jobs.data()), t.fj.jobs.size() / 2);
+    geom.upload(t.geom.data(), t.geom.size());
     ipr.upload(t.fj.ipr.data(), t.fj.ipr.size());
     MXM_HIP(hipDeviceSynchronize());
   }
@@ -237,10 +238,10 @@ struct Solver {
     a.a = pl.a, a.b = pl.b, a.c = pl.c;
     a.inst_prm = dprm.p;  // one instance: tile_inst, inst_dt, inst_post, inst_active stay null
     a.dt = dt;
-    a.tile_count = tile_count.p;
-    a.invJ = invJ.p, a.inv_vol = inv_vol.p;
+    a.tile_count = tile_count.p, a.tile_type = tile_type.p;
+    a.geom = geom.p;
     a.Dt = Dt.p, a.Lt = Lt.p, a.Aop = Aop.p, a.fmap = fmap.p;
-    a.jobs = jobs.p, a.jgeo = jgeo.p, a.ipr = ipr.p, a.maxj = maxj, a.ntiles = ntiles;
+    a.jobs = jobs.p, a.ipr = ipr.p, a.maxj = maxj, a.ntiles = ntiles;
     a.post_comp = s == 2 ? post_component(phys, prm) : -1;
     a.post_scale = post_factor(phys, prm, dt);
     // limiter: the stage epilogue writes the output's cell means and node
@@ -848,7 +849,7 @@ int mxm_dg_memory_report(void *h, mxm_memory_report *o) {
     o->dg_operators = (long long)(s->Dt.bytes() + s->Lt.bytes() + s->Aop.bytes() + s->w.bytes() + s->fmap.bytes());
     o->limiter = (long long)(s->lmean.bytes() + s->ltheta.bytes() + s->lext.bytes());
     o->mesh_connectivity = (long long)(s->invJ.bytes() + s->inv_vol.bytes() + s->conn.bytes() +
-                                       s->jgeo.bytes() + s->jobs.bytes() + s->ipr.bytes() +
+                                       s->geom.bytes() + s->tile_type.bytes() + s->jobs.bytes() + s->ipr.bytes() +
                                        s->tile_count.bytes());
     o->halo_device = 0;
     o->halo_pinned = 0;

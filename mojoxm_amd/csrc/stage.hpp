@@ -45,6 +45,7 @@
 
 #include <type_traits>
 
+#include "host.hpp"
 #include "physics.hpp"
 
 namespace mxm {
@@ -80,15 +81,16 @@ struct StageArgs {
   double dt, post_scale;
   int post_comp;            // component scaled after the combine (GLM psi), -1 none
   const int *tile_count;  // [ntiles] elements in each tile (slots T*EPB ..)
-  const double *invJ;     // [slots][ND*ND] rows = reference directions
-  const double *inv_vol;  // [slots] 1/(6V) or 1/(2A)
+  const double *geom;     // [n_inst][stage_geom_len]: the mesh's distinct face normals and areas
+                          // ([max_face_geo][4]), then per element of a lattice cell invJ (ND*ND, rows =
+                          // reference directions) and inv_vol (1/(6V) or 1/(2A))
+  const int *tile_type;   // [ntiles] cell element of the tile's first slot
   const double *Dt;       // FP64 form: [ND*NP (k,j)][NPAD (i)] transposed D_ref, zero padded
   const double *Lt;       // FP64 form: [NF*NFP (f,r)][NPAD (i)] transposed Lift_ref, zero padded
   const float *Aop;       // FP32 form: [16*MT (i)][KPAD (k)] = [D_0 .. D_ND-1 | Lift], zero padded
   const int *fmap;        // [NF][NFP] element node of each reference face slot
-  const int4 *jobs;       // [ntiles*maxj] {el | lf<<7 | pin<<9 | plf<<16 | pslot<<18
-                          //  (-1: padding), partner slot, face id, side | bc<<1}
-  const double *jgeo;     // [ntiles*maxj][4] face normal, area
+  const int2 *jobs;       // [ntiles*maxj] {el | lf<<7 | pin<<9 | plf<<16 | side<<18 | bc<<19 | geometry<<22
+                          //  (-1: padding), partner slot}
   const unsigned short *ipr;  // [ntiles*maxj*NFP] partner node | partner slot << 8
   int maxj;               // job slots per tile
   int ntiles;
@@ -148,6 +150,7 @@ constexpr int stage_lds_bytes(int ND, int NP, int NFP, int NC, int epb) {
               : ND * NP * (epb * NC + 1)) * 8 +
          epb * (ND * ND + 1) * 8 + (ND + 1) * NFP * 4;
 }
+constexpr int stage_geom_len(int ND) { return 4 * max_face_geo(ND) + cell_elems(ND) * (ND * ND + 1); }
 constexpr int stage_epb(int ND, int NP, int NFP, int NC, bool wide = false) {
   const int cell = ND == 3 ? 6 : 2;
   int e = 256 / NP;
@@ -231,12 +234,9 @@ __device__ __forceinline__ int xcd_tile(int bid, int nb) {
 // that follow.
 template <class R, int NC>
 struct FaceItem {
-  int4 job;        // StageArgs::jobs
-  double2 g0, g1;  // normal x, y | normal z, area
-  unsigned pr;     // StageArgs::ipr
-  R qp[NC];        // partner trace when the partner is outside the tile
-  __device__ __forceinline__ int side() const { return job.w & 1; }
-  __device__ __forceinline__ int bc() const { return (job.w >> 1) & 7; }
+  int2 job;     // StageArgs::jobs
+  unsigned pr;  // StageArgs::ipr
+  R qp[NC];     // partner trace when the partner is outside the tile
 };
 
 // A value of the state with its element's pending limiter factor applied:
@@ -270,13 +270,10 @@ __device__ __forceinline__ int small_div(int x) {
 // trace of a face to another tile is the only load that waits for one of
 // them (load_item_trace).
 template <int NFP, int MAXT, class R, int NC>
-__device__ __forceinline__ void load_item_records(const int4 *jobs, const double *jgeo, const unsigned short *ipr,
-                                                  int t, FaceItem<R, NC> &it) {
-  const int jb = small_div<NFP, MAXT>(t);
-  it.job = jobs[jb];
+__device__ __forceinline__ void load_item_records(const int2 *jobs, const unsigned short *ipr, int t,
+                                                  FaceItem<R, NC> &it) {
+  it.job = jobs[small_div<NFP, MAXT>(t)];
   it.pr = ipr[t];
-  it.g0 = reinterpret_cast<const double2 *>(jgeo)[2 * jb];
-  it.g1 = reinterpret_cast<const double2 *>(jgeo)[2 * jb + 1];
 }
 
 // A partner slot in the tile's own range is in the tile: partners are real
@@ -387,7 +384,16 @@ dg_stage_kernel(StageArgs<R> A) {
   // [el][i][c].  sS = sB + TILE: face fluxes [f*NFP + r][el][c].
   __shared__ __align__(16) R sB[NB];
   __shared__ float sA[kStageA ? MT * 16 * KAS : 1];
-  __shared__ double sJ[EPB * ND * ND + EPB];  // invJ then inv_vol
+  // the geometry (StageArgs::geom): face normals and areas, then invJ and
+  // inv_vol of each element of a lattice cell.  A lattice has a handful of
+  // each, so a tile reads 0.2 to 1 KB for them, the same for every tile,
+  // where a record per face and per slot took 3 KB: 77 of the 251 MB that
+  // the FP32 512^2 vortex stage fetched (90.6 -> 86.0 us; 32^3 Taylor-Green
+  // FP64 186 -> 181, 16^3 P = 2 advection 7.9 -> 7.5).
+  constexpr int EPC = cell_elems(ND), GEL = ND * ND + 1, GEOM = stage_geom_len(ND);
+  static_assert(GEOM <= 256, "one geometry value per thread");
+  __shared__ __align__(16) double sG[GEOM];
+  const double *const sE = sG + 4 * max_face_geo(ND);
   __shared__ int sMap[NF * NFP];
   // pending limiter factors of the tile's elements, then their means (q_in)
   constexpr int NL = EPB * (NC + 1);
@@ -419,16 +425,13 @@ dg_stage_kernel(StageArgs<R> A) {
   typedef R TileVec __attribute__((ext_vector_type(VW)));
   constexpr int TV = TILE / VW;
   constexpr int QPT = (TV + S::BLOCK - 1) / S::BLOCK;     // tile vectors per thread
-  constexpr int NJ = EPB * ND * ND, NG = NJ + EPB;        // invJ, then inv_vol
-  constexpr int GPT = (NG + S::BLOCK - 1) / S::BLOCK;
   constexpr int MAXT = EPB * NFF;                         // face items of a tile, at most
   const size_t tile0 = (size_t)tile * TILE;               // the tile's first value
   const size_t job0 = (size_t)tile * A.maxj;
-  const int4 *const jobs = A.jobs + job0;
-  const double *const jgeo = A.jgeo + 4 * job0;
+  const int2 *const jobs = A.jobs + job0;
   const unsigned short *const ipr = A.ipr + NFP * job0;
   FaceItem<R, NC> it;
-  load_item_records<NFP, MAXT>(jobs, jgeo, ipr, tid < nitems ? tid : nitems - 1, it);
+  load_item_records<NFP, MAXT>(jobs, ipr, tid < nitems ? tid : nitems - 1, it);
   const TileVec *const src = reinterpret_cast<const TileVec *>(A.q_in + tile0);
   TileVec tq[QPT];
 #pragma unroll
@@ -456,17 +459,6 @@ dg_stage_kernel(StageArgs<R> A) {
       for (int c = 0; c < NC; ++c) qa_in[c] = g[c];
     }
   }
-  double tg[GPT];
-  {
-    const double *const gj = A.invJ + (size_t)tile * NJ, *const gv = A.inv_vol + e0;
-#pragma unroll
-    for (int k = 0; k < GPT; ++k) {
-      int t = k * S::BLOCK + tid;
-      t = (k + 1) * S::BLOCK <= NG || t < NG ? t : NG - 1;
-      const double *g = t < NJ ? gj + t : gv + (t - NJ);
-      tg[k] = *g;
-    }
-  }
   const int fm = A.fmap[tid < NFF ? tid : NFF - 1];
   constexpr int APT = kStageA ? (NA + S::BLOCK - 1) / S::BLOCK : 0;
   float ta[APT > 0 ? APT : 1];
@@ -490,7 +482,9 @@ dg_stage_kernel(StageArgs<R> A) {
     }
   }
   const int nE = A.tile_count[tile];
+  const int type0 = EPB % EPC ? A.tile_type[tile] : 0;
   const int inst = A.tile_inst ? A.tile_inst[tile] : 0;
+  const double tg = A.geom[(size_t)inst * GEOM + (tid < GEOM ? tid : GEOM - 1)];
   // the instance's switch, parameters and step
   const int on = A.inst_active ? A.inst_active[inst] : 1;
   const Phys phys = Phys::from(A.inst_prm + (size_t)inst * kPrmMax);
@@ -512,11 +506,7 @@ dg_stage_kernel(StageArgs<R> A) {
     const int t = k * S::BLOCK + tid;
     if ((k + 1) * S::BLOCK <= TV || t < TV) reinterpret_cast<TileVec *>(sW)[t] = tq[k];
   }
-#pragma unroll
-  for (int k = 0; k < GPT; ++k) {
-    const int t = k * S::BLOCK + tid;
-    if (t < NG) sJ[t] = tg[k];
-  }
+  if (tid < GEOM) sG[tid] = tg;
   if (tid < NFF) sMap[tid] = fm;
   if constexpr (kQaLds) {
     if (!qa_is_in) {
@@ -559,6 +549,13 @@ dg_stage_kernel(StageArgs<R> A) {
     __syncthreads();
   }
   const R *sQ = sW;  // the q_in tile, [el][j][c], until the flux planes are written
+  // element el's place in its lattice cell
+  auto cell_type = [&](int el) {
+    if constexpr (EPB % EPC == 0)
+      return el - small_div<EPC, 128>(el) * EPC;
+    else
+      return type0 + el - small_div<EPC, 128>(type0 + el) * EPC;
+  };
 
   // ---- 2a. face fluxes ----------------------------------------------------
   // Both states of an item are read from LDS by offset: a trace that came
@@ -567,11 +564,13 @@ dg_stage_kernel(StageArgs<R> A) {
   // the left one is then a choice between two offsets.
   for (int t = tid; t < nitems; t += S::BLOCK) {
     if (t != tid) {
-      load_item_records<NFP, MAXT>(jobs, jgeo, ipr, t, it);
+      load_item_records<NFP, MAXT>(jobs, ipr, t, it);
       load_item_trace<NP, EPB, LIM>(A, e0, it);
     }
     if (it.job.x < 0) continue;
     const int el = it.job.x & 127, lf = (it.job.x >> 7) & 3, pin = (it.job.x >> 9) & 127;
+    const int bc = (it.job.x >> 19) & 7;
+    const double *const geo = sG + 4 * (it.job.x >> 22);  // normal, area
     const int fr = lf * NFP + (t - small_div<NFP, MAXT>(t) * NFP);
     const int pl = it.job.y - e0, slot = TILE + fr * NCOLS + el * NC;
     const int mine = (el * NP + sMap[fr]) * NC;
@@ -582,28 +581,28 @@ dg_stage_kernel(StageArgs<R> A) {
       for (int c = 0; c < NC; ++c) sB[slot + c] = it.qp[c];
     }
     // left = side-0 trace; right = side-1 trace or the ghost of the left
-    const bool s0 = it.side() == 0;
+    const bool s0 = !(it.job.x & (1 << 18));
     const R *const pL = sB + (s0 ? mine : other), *const pR = sB + (s0 ? other : mine);
-    const R n[3] = {R(it.g0.x), R(it.g0.y), R(it.g1.x)};
+    const R n[3] = {R(geo[0]), R(geo[1]), ND == 3 ? R(geo[2]) : R(0)};
     R ql[NC], qr[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) ql[c] = pL[c];
-    if (it.bc())
-      phys.ghost(ql, it.bc(), n, qr);
+    if (bc)
+      phys.ghost(ql, bc, n, qr);
     else
 #pragma unroll
       for (int c = 0; c < NC; ++c) qr[c] = pR[c];
     R Fs[NC];
     phys.template numerical_flux<ND>(ql, qr, n, Fs);
-    const double sa = s0 ? it.g1.y : -it.g1.y;
+    const double sa = s0 ? geo[3] : -geo[3];
     // FP64 form: s area F*, lifted and scaled by -inv_vol in the
     // contraction; FP32 form: -inv_vol s area F*, ready for the product
-    const R own = kMFMA ? R(-sJ[EPB * ND * ND + el] * sa) : R(sa);
+    const R own = kMFMA ? R(-sE[cell_type(el) * GEL + ND * ND] * sa) : R(sa);
 #pragma unroll
     for (int c = 0; c < NC; ++c) sB[slot + c] = own * Fs[c];
     if (pin) {
       const int plf = (it.job.x >> 16) & 3, rs = it.pr >> 8;
-      const R oth = kMFMA ? R(sJ[EPB * ND * ND + pin - 1] * sa) : R(-sa);
+      const R oth = kMFMA ? R(sE[cell_type(pin - 1) * GEL + ND * ND] * sa) : R(-sa);
 #pragma unroll
       for (int c = 0; c < NC; ++c) sS[(plf * NFP + rs) * NCOLS + (pin - 1) * NC + c] = oth * Fs[c];
     }
@@ -619,7 +618,7 @@ dg_stage_kernel(StageArgs<R> A) {
     const R *q = &sQ[tid * NC];
     R F[ND * NC];
     phys.template flux<ND>(q, F);
-    const double *iJ = &sJ[nel * ND * ND];
+    const double *iJ = sE + cell_type(nel) * GEL;
     if constexpr (kMFMA) {
       // FP32 form: the mapping in FP32 (invJ rounded once per node), as
       // the volume product that takes its result is
@@ -743,7 +742,7 @@ dg_stage_kernel(StageArgs<R> A) {
 #pragma unroll
           for (int ii = 0; ii < IH; ++ii) dacc[m][ii] += L[ii] * sv;
         }
-        const double niv = -sJ[EPB * ND * ND + el];
+        const double niv = -sE[cell_type(el) * GEL + ND * ND];
 #pragma unroll
         for (int ii = 0; ii < IH; ++ii) dacc[m][ii] *= niv;
       }
