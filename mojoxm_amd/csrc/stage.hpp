@@ -97,6 +97,12 @@ struct StageArgs {
 };
 
 constexpr int kPrmMax = 32;  // MXM_PRM_MAX
+// FP64 operators up to this size are read into the scalar cache (16 KB for
+// two CUs) by the first blocks of a launch, one or so per CU
+constexpr int kScalarWarmBytes = 4096, kScalarWarmBlocks = 256;
+// read-only data in the constant address space: wave-uniform loads stay scalar
+// whatever stands between them
+typedef const double __attribute__((address_space(4))) *ScalarPtr;
 
 // Launch configurations of the stage kernel: each is an occupancy target
 // (waves per SIMD, e.g. 256-thread blocks per CU) that bounds the register
@@ -492,6 +498,30 @@ dg_stage_kernel(StageArgs<R> A) {
   const double post = A.inst_post ? A.inst_post[inst] : A.post_scale;
   if (!on) return;
   load_item_trace<NP, EPB, LIM>(A, e0, it);
+  // FP64 form: the contraction streams the operator through the scalar
+  // cache, which every launch starts with cold, a few rows at a time: a
+  // chain of misses.  The launch's first blocks touch each line of a small
+  // operator here, all at once and behind the tile's own loads (48^2 GLM-MHD
+  // 7.5 -> 6.6 us, 33^2 P = 2 Euler 5.5 -> 5.1); done by every block, or for
+  // operators beyond 4 KB, it cost more than it saved (16^3 P = 2 advection
+  // 6.4 -> 7.7 us).
+  if constexpr (!kMFMA) {
+    constexpr int WAVES = S::BLOCK / 64, WORDS = stage_node_pad(EPB, NP, NC) * 2;
+    constexpr int LD = (KV * WORDS + 15) / 16, LINES = LD + (NFF * WORDS + 15) / 16, LPW = (LINES + WAVES - 1) / WAVES;
+    if (LINES * 64 <= kScalarWarmBytes && blockIdx.x < kScalarWarmBlocks) {
+      typedef const unsigned __attribute__((address_space(4))) *Line;
+      const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+      unsigned x[LPW], any = 0;
+#pragma unroll
+      for (int k = 0; k < LPW; ++k) {
+        const int line = k * WAVES + w < LINES ? k * WAVES + w : LINES - 1;
+        x[k] = line < LD ? ((Line)A.Dt)[line * 16] : ((Line)A.Lt)[(line - LD) * 16];
+      }
+#pragma unroll
+      for (int k = 0; k < LPW; ++k) any |= x[k];
+      asm volatile("" ::"s"(any));
+    }
+  }
   // thread tid owns output node (el, i) = (tid / NP, tid % NP): EPB*NP <= BLOCK
   const int nel = small_div<NP, S::BLOCK>(tid), nod = tid - nel * NP;
   const bool node = tid < nE * NP;
@@ -692,6 +722,65 @@ dg_stage_kernel(StageArgs<R> A) {
   const int lane = tid - grp * GSIZE;
   double dacc[kMFMA ? 1 : ITER][kMFMA ? 1 : IH];
 
+  // acc[ii] += sum_r op[r][ii] col[r] over N rows: RB rows at a time, the next
+  // rows' scalar and LDS loads in flight behind the FMAs of the present ones
+  // (two sets of RB*IH <= 16 operator entries in scalar registers).  Scalar
+  // loads return out of order, so a wait for some is a wait for all: it
+  // stands before the next rows are asked for.  Against one set, loaded and
+  // waited for, us per stage: 512^2 vortex 149.7 -> 145.4, 128^2 14.1 -> 13.7,
+  // 32^3 Taylor-Green 181 -> 176.5, 16^3 P = 2 advection 7.5 -> 6.7.
+  [[maybe_unused]] auto contract = [&](const R *col, ScalarPtr op, auto N, double (&acc)[kMFMA ? 1 : IH]) {
+    constexpr int RB = IH <= 16 ? 16 / IH : 1, SETS = (N + RB - 1) / RB;
+    double o[2][RB][IH], v[2][RB];
+    auto load = [&](int b, int s) {
+#pragma unroll
+      for (int r = 0; r < RB; ++r) {
+        const int row = b * RB + r < N ? b * RB + r : N - 1;  // past the end: loaded, not used
+        v[s][r] = col[row * NCOLS];
+#pragma unroll
+        for (int ii = 0; ii < IH; ++ii) o[s][r][ii] = op[row * NPAD + ii];
+      }
+    };
+    auto use = [&](int s, int n) {
+#pragma unroll
+      for (int r = 0; r < RB; ++r)
+        if (r < n) {
+#pragma unroll
+          for (int ii = 0; ii < IH; ++ii) acc[ii] += o[s][r][ii] * v[s][r];
+        }
+    };
+    auto arrived = [] {
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // short products in full (16^3 P = 2 advection 8.0 -> 6.7 us); long ones
+    // as a loop, which costs them nothing
+    constexpr int pairs = N * IH <= 100 ? SETS : 1;
+    load(0, 0);
+#pragma unroll pairs
+    for (int b = 0; b + 2 < SETS; b += 2) {
+      arrived();
+      load(b + 1, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      use(0, RB);
+      arrived();
+      load(b + 2, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      use(1, RB);
+    }
+    // the last set or two
+    constexpr int left = SETS % 2 ? 1 : 2, last = N - (SETS - 1) * RB;
+    arrived();
+    if constexpr (left == 2) {
+      load(SETS - 1, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      use(0, RB);
+      arrived();
+      use(1, last);
+    } else {
+      use(0, last);
+    }
+  };
   // one 4-deep step of the MFMA product over operator columns k0.. and
   // operand rows kb.. of Bb
   auto kstep = [&](const R *Bb, int k0, int kb) {
@@ -735,13 +824,7 @@ dg_stage_kernel(StageArgs<R> A) {
       for (int ii = 0; ii < IH; ++ii) dacc[m][ii] = 0.0;
       if (p < nE * NC) {
         const int el = small_div<NC, ITER * GSIZE>(p);
-#pragma unroll 4
-        for (int fr = 0; fr < NFF; ++fr) {
-          const double sv = sS[fr * NCOLS + p];
-          const double *L = A.Lt + fr * NPAD + i0;
-#pragma unroll
-          for (int ii = 0; ii < IH; ++ii) dacc[m][ii] += L[ii] * sv;
-        }
+        contract(sS + p, (ScalarPtr)A.Lt + i0, std::integral_constant<int, NFF>{}, dacc[m]);
         const double niv = -sE[cell_type(el) * GEL + ND * ND];
 #pragma unroll
         for (int ii = 0; ii < IH; ++ii) dacc[m][ii] *= niv;
@@ -792,13 +875,7 @@ dg_stage_kernel(StageArgs<R> A) {
     for (int m = 0; m < ITER; ++m) {
       const int p = lane + m * GSIZE;
       if (p < nE * NC) {
-#pragma unroll 4
-        for (int kj = 0; kj < KV; ++kj) {
-          const double fv = sW[kj * NCOLS + p];
-          const double *D = A.Dt + kj * NPAD + i0;
-#pragma unroll
-          for (int ii = 0; ii < IH; ++ii) dacc[m][ii] += D[ii] * fv;
-        }
+        contract(sW + p, (ScalarPtr)A.Dt + i0, std::integral_constant<int, KV>{}, dacc[m]);
       }
     }
     __syncthreads();
