@@ -94,9 +94,9 @@ using GroupKey = std::tuple<int, int, int, int, int, long long>;  // dim, P, phy
 struct Arena {
   DevBuf<double> qd[3];
   DevBuf<float> qf[3];
-  // limiter (groups with it): cell means [3][slots*NC] and factors
-  // [3][slots] of the stage buffers, node extrema [slots*NCL][2] (the
-  // limited components: all NC in 3D, component 0 in 2D)
+  // limiter (groups with it): cell means [3][slots*NC], node extrema
+  // [3][slots*NCL][2] (the limited components: all NC in 3D, component 0 in
+  // 2D) and factors [3][slots] of the stage buffers
   DevBuf<double> lmean, ltheta, lext;
   DevBuf<double> invJ, inv_vol, geom, iprm, idt, ipost;  // geom: one table per instance slot
   DevBuf<int> conn;  // limiter: partner slot per face
@@ -244,7 +244,7 @@ size_t instance_bytes(const ElemTables &t, int NP, int NC, int NFP, int dim, int
   b += js * (sizeof(int2) + NFP * sizeof(unsigned short));          // jobs, partner nodes
   b += tiles * 3 * sizeof(int);                                     // tile_count, tile_type, tile_inst
   b += (MXM_PRM_MAX + 2 + t.geom.size()) * sizeof(double) + 4 * sizeof(int);  // per-instance scalars, geometry
-  if (limiter) b += slots * (3 * NC + 2 * (dim == 3 ? NC : 1) + 3) * sizeof(double);  // means, factors, extrema
+  if (limiter) b += slots * (3 * NC + 6 * (dim == 3 ? NC : 1) + 3) * sizeof(double);  // means, factors, extrema
   return b;
 }
 
@@ -472,13 +472,14 @@ struct Batch {
   void materialize(BGroup &g, int s0, int n) {
     const size_t S = g.ar.ltheta.n / 3;
     if (n <= 0 || (size_t)s0 + n > S) return;
-    const size_t vo = (size_t)s0 * g.NP * g.NC;
+    auto limit = [&](auto *q) {
+      MXM_HIP(launch_bj_limit(q, g.ar.ltheta.p, g.ar.lmean.p, g.ar.lext.p, g.ar.conn.p, s0, n, g.NP, g.NC, g.NF, g.dim,
+                              g.eps, g.stream));
+    };
     if (g.prec == MXM_PREC_FP64)
-      MXM_HIP(launch_bj_apply<double>(g.ar.qd[0].p + vo, g.ar.ltheta.p + s0, g.ar.lmean.p + (size_t)s0 * g.NC, n,
-                                      g.NP, g.NC, g.stream));
+      limit(g.ar.qd[0].p);
     else
-      MXM_HIP(launch_bj_apply<float>(g.ar.qf[0].p + vo, g.ar.ltheta.p + s0, g.ar.lmean.p + (size_t)s0 * g.NC, n,
-                                     g.NP, g.NC, g.stream));
+      limit(g.ar.qf[0].p);
   }
 
   // ---- staging ----------------------------------------------------------
@@ -537,10 +538,10 @@ struct Batch {
     }
     hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, g.stream, g.ar.ifail.p + sl, 0, 1);
     MXM_HIP(hipGetLastError());
-    if (g.limiter) {  // nothing pending on the new state (the range may hold a removed instance's factors)
-      const size_t S = g.ar.ltheta.n / 3;
-      for (int b = 0; b < 3; ++b)
-        MXM_HIP(launch_fill(g.ar.ltheta.p + b * S + bs, (long long)in.ntiles() * g.epb, 1.0, g.stream));
+    if (g.limiter) {  // nothing pending on the new state (the range may hold a removed instance's extrema)
+      const size_t n = (size_t)in.ntiles() * g.epb, ncl = g.dim == 3 ? g.NC : 1;
+      MXM_HIP(launch_fill(g.ar.lmean.p + bs * g.NC, (long long)(n * g.NC), 0.0, g.stream));
+      MXM_HIP(launch_fill(g.ar.lext.p + bs * ncl * 2, (long long)(n * ncl * 2), 0.0, g.stream));
     }
     MXM_HIP(hipEventRecord(st.ev, g.stream));
     st.busy = true;
@@ -701,8 +702,10 @@ struct Batch {
     na.ifail.upload(ifl.data(), ifl.size());
     if (g.limiter) {
       na.lmean.alloc(3 * slots * g.NC);
-      na.lext.alloc(2 * slots * (g.dim == 3 ? g.NC : 1));
+      na.lext.alloc(3 * 2 * slots * (g.dim == 3 ? g.NC : 1));
       na.ltheta.alloc(3 * slots);
+      MXM_HIP(launch_fill(na.lmean.p, (long long)na.lmean.n, 0.0, g.stream));
+      MXM_HIP(launch_fill(na.lext.p, (long long)na.lext.n, 0.0, g.stream));
       MXM_HIP(launch_fill(na.ltheta.p, (long long)na.ltheta.n, 1.0, g.stream));
     }
     // ---- commit (no more allocations or copies that can fail) ----
@@ -790,10 +793,12 @@ struct Batch {
     a.inst_active = ar.iactive.p;
     a.inst_fail = ar.ifail.p;
     if (g.limiter) {  // as in the solver: outputs' means and extrema, inputs' pending factors
-      const size_t S = ar.ltheta.n / 3, kn = S * g.NC;
-      a.mean = ar.lmean.p + pl.out * kn, a.ext = ar.lext.p;
-      a.lim_th_in = ar.ltheta.p + pl.in * S, a.lim_mn_in = ar.lmean.p + pl.in * kn;
+      const size_t S = ar.ltheta.n / 3, kn = S * g.NC, kx = S * (g.dim == 3 ? g.NC : 1) * 2;
+      a.mean = ar.lmean.p + pl.out * kn, a.ext = ar.lext.p + pl.out * kx;
+      a.lim_mn_in = ar.lmean.p + pl.in * kn, a.lim_ext_in = ar.lext.p + pl.in * kx;
+      a.lim_th_in = ar.ltheta.p + pl.in * S;
       a.lim_th_a = ar.ltheta.p + pl.qa * S, a.lim_mn_a = ar.lmean.p + pl.qa * kn;
+      a.conn = ar.conn.p, a.lim_eps2 = g.eps * g.eps;
     }
     a.w = g.w.p;
     a.dt = 0.0, a.post_scale = 1.0;
@@ -811,10 +816,6 @@ struct Batch {
     for (int st = 0; st < 3; ++st) {
       const StageArgs<R> a = stage_args(g, q, st);
       MXM_HIP(g.launch(&a, s));
-      if (g.limiter)
-        MXM_HIP(launch_bj_theta(g.ar.ltheta.p + (g.ar.ltheta.n / 3) * stage_plan(st).out, a.mean, g.ar.lext.p,
-                                g.ar.conn.p, g.grid_tiles * g.epb, g.NC, g.NF, g.dim, g.eps, s, g.ar.tile_count.p,
-                                g.epb, g.ar.tile_inst.p, g.ar.iactive.p));
     }
     // over every slot of the arena (later placements need no recapture;
     // slots not in use are inactive)

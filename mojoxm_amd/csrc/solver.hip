@@ -58,9 +58,9 @@ struct Solver {
   // state trio q, q1, q2: FP64 (MXM_PREC_FP64) or FP32 (MXM_PREC_FP32_MFMA)
   DevBuf<double> q, q1, q2;
   DevBuf<float> f, f1, f2;
-  // limiter: cell means [3][Kd*NC] and factors [3][Kd] of the stage
-  // buffers (q, q1, q2), node extrema [Kd*NCL][2] of the last stage output
-  // (the limited components: all NC in 3D, component 0 in 2D)
+  // limiter: cell means [3][Kd*NC], node extrema [3][Kd*NCL][2] (the limited
+  // components: all NC in 3D, component 0 in 2D) and factors [3][Kd] of the
+  // stage buffers (q, q1, q2)
   DevBuf<double> lmean, ltheta, lext;
   DevBuf<double> invJ, inv_vol, geom, Dt, Lt, w, dprm;
   DevBuf<double> Dn, dpart, dout;  // diagnostics: nodal derivative, tile partials, results
@@ -142,6 +142,14 @@ struct Solver {
     }
   }
 
+  // components the limiter bounds
+  int ncl() const { return dim == 3 ? NC : 1; }
+  // nothing pending: extrema equal to the means, factors 1
+  void clear_pending() {
+    MXM_HIP(launch_fill(lmean.p, (long long)lmean.n, 0.0, stream));
+    MXM_HIP(launch_fill(lext.p, (long long)lext.n, 0.0, stream));
+    MXM_HIP(launch_fill(ltheta.p, (long long)ltheta.n, 1.0, stream));
+  }
   bool has_wide() const { return prec == MXM_PREC_FP32_MFMA && stage_has_wide(dim, NP, NFP, NC); }
   StageLaunch find(int c, bool lim) const { return find_stage(dim, phys, variant, P, prec, c, lim, wide); }
 
@@ -166,9 +174,9 @@ struct Solver {
       }
     }
     lmean.alloc((size_t)3 * Kd * NC);
-    lext.alloc((size_t)2 * Kd * (dim == 3 ? NC : 1));  // the limited components only
+    lext.alloc((size_t)3 * 2 * Kd * ncl());
     ltheta.alloc((size_t)3 * Kd);
-    MXM_HIP(launch_fill(ltheta.p, (long long)ltheta.n, 1.0, stream));
+    clear_pending();
     invJ.upload(t.invJ.data(), t.invJ.size());
     inv_vol.upload(t.inv_vol.data(), t.inv_vol.size());
     conn.upload(t.conn.data(), t.conn.size());
@@ -189,7 +197,7 @@ struct Solver {
   static constexpr double kWarmUpMs = 30.0;
   void warm_up(double dt, double ms) {
     const auto t0 = std::chrono::steady_clock::now();
-    for (int k = 1, total = 0; total < 65536; total += k, k = k < 256 ? 2 * k : 256) {
+    for (int k = 1, total = 0; total < 65536; total += k, k = k < 32 ? 2 * k : 32) {
       for (int j = 0; j < k; ++j)
         for (int st = 0; st < 3; ++st) stage(st, dt);
       MXM_HIP(hipStreamSynchronize(stream));
@@ -245,13 +253,15 @@ struct Solver {
     a.post_comp = s == 2 ? post_component(phys, prm) : -1;
     a.post_scale = post_factor(phys, prm, dt);
     // limiter: the stage epilogue writes the output's cell means and node
-    // extrema, the theta kernel its factors; the inputs' pending factors
-    // are applied as they are read
+    // extrema; the inputs' pending factors are computed and applied as they
+    // are read
     if (limiter) {
-      const size_t kn = (size_t)Kd * NC;
-      a.mean = lmean.p + pl.out * kn, a.ext = lext.p;
-      a.lim_th_in = ltheta.p + (size_t)pl.in * Kd, a.lim_mn_in = lmean.p + pl.in * kn;
+      const size_t kn = (size_t)Kd * NC, kx = (size_t)Kd * ncl() * 2;
+      a.mean = lmean.p + pl.out * kn, a.ext = lext.p + pl.out * kx;
+      a.lim_mn_in = lmean.p + pl.in * kn, a.lim_ext_in = lext.p + pl.in * kx;
+      a.lim_th_in = ltheta.p + (size_t)pl.in * Kd;
       a.lim_th_a = ltheta.p + (size_t)pl.qa * Kd, a.lim_mn_a = lmean.p + pl.qa * kn;
+      a.conn = conn.p, a.lim_eps2 = eps * eps;
     }
     a.w = w.p;
     return a;
@@ -261,26 +271,24 @@ struct Solver {
   void stage_with(int s, double dt, R *b0, R *b1, R *b2) {
     const StageArgs<R> a = stage_args(s, dt, b0, b1, b2);
     MXM_HIP(kernel()(&a, stream));
-    if (limiter)
-      MXM_HIP(launch_bj_theta(ltheta.p + (size_t)stage_plan(s).out * Kd, a.mean, lext.p, conn.p, Kd, NC, NF, dim,
-                              eps, stream, tile_count.p, til.epb));
   }
 
   // the stage kernel of the launch configuration, in its limited variant
   // when the limiter is on
   StageLaunch kernel() const { return limiter ? find(cfg, true) : launch; }
 
-  // writes the limited values of stage buffer b (0 = q) and clears its
-  // pending factors
+  // writes the limited values of stage buffer b (0 = q); nothing is pending
+  // on it afterwards
   void materialize(int b) {
-    const size_t kn = (size_t)Kd * NC;
-    if (prec == MXM_PREC_FP64) {
-      double *t[3] = {q.p, q1.p, q2.p};
-      MXM_HIP(launch_bj_apply<double>(t[b], ltheta.p + (size_t)b * Kd, lmean.p + b * kn, Kd, NP, NC, stream));
-    } else {
-      float *t[3] = {f.p, f1.p, f2.p};
-      MXM_HIP(launch_bj_apply<float>(t[b], ltheta.p + (size_t)b * Kd, lmean.p + b * kn, Kd, NP, NC, stream));
-    }
+    const size_t kn = (size_t)Kd * NC, kx = (size_t)Kd * ncl() * 2;
+    auto limit = [&](auto *t) {
+      MXM_HIP(launch_bj_limit(t, ltheta.p + (size_t)b * Kd, lmean.p + b * kn, lext.p + b * kx, conn.p, 0, Kd, NP, NC,
+                              NF, dim, eps, stream));
+    };
+    if (prec == MXM_PREC_FP64)
+      limit(b == 0 ? q.p : b == 1 ? q1.p : q2.p);
+    else
+      limit(b == 0 ? f.p : b == 1 ? f1.p : f2.p);
   }
 
   // times every launch configuration of the current tiling on SSPRK3
@@ -458,7 +466,7 @@ struct Solver {
         for (size_t k = 0; k < node; ++k) d[(size_t)til.dev_of[e] * node + k] = float(h[(size_t)e * node + k]);
       MXM_HIP(hipMemcpy(f.p, d.data(), n * sizeof(float), hipMemcpyHostToDevice));
     }
-    MXM_HIP(launch_fill(ltheta.p, (long long)ltheta.n, 1.0, stream));  // nothing pending on a new state
+    clear_pending();
   }
   void download_state(double *h) {
     const size_t node = (size_t)NP * NC, n = (size_t)Kd * node;

@@ -45,6 +45,7 @@
 
 #include <type_traits>
 
+#include "bj.hpp"
 #include "host.hpp"
 #include "physics.hpp"
 
@@ -72,12 +73,17 @@ struct StageArgs {
   double *ext;              // [slots][NCL][2] (with mean): smallest and largest stored node value of the
                             // limited components (all NC in 3D, component 0 in 2D)
   const double *w;          // [NP] node weights (with mean)
-  // Limiter factors pending on the input buffers (nullptr: none): every
-  // value read from q_in (tile and partner traces) or q_a is used as
-  // mean + theta (q - mean) where its element's theta < 1, which is the
-  // state the limiter would have stored.
-  const double *lim_th_in, *lim_mn_in;  // q_in: theta [slots], means [slots][NC]
-  const double *lim_th_a, *lim_mn_a;    // q_a
+  // Limiter (mean != nullptr).  The factors pending on q_in are computed
+  // from its means and node extrema as it is read (extrema equal to the means:
+  // nothing pending) and stored; q_a's are those that stage 1 stored.  A value
+  // read from q_in (tile and partner traces) or q_a is used as
+  // mean + theta (q - mean) where its element's theta < 1, which is the state
+  // the limiter would have stored.
+  const double *lim_mn_in, *lim_ext_in;  // q_in: means [slots][NC], extrema [slots][NCL][2]
+  double *lim_th_in;                     // q_in: theta [slots], written for the tile's elements
+  const double *lim_th_a, *lim_mn_a;     // q_a: theta, means
+  const int *conn;                       // [slots][NF] partner slot of each face
+  double lim_eps2;                       // Venkatakrishnan's eps^2
   double dt, post_scale;
   int post_comp;            // component scaled after the combine (GLM psi), -1 none
   const int *tile_count;  // [ntiles] elements in each tile (slots T*EPB ..)
@@ -244,6 +250,11 @@ struct FaceItem {
   unsigned pr;  // StageArgs::ipr
   R qp[NC];     // partner trace when the partner is outside the tile
 };
+// the partner's cell means (limited kernels)
+template <int NC>
+struct FaceMeans {
+  double m[NC];
+};
 
 // A value of the state with its element's pending limiter factor applied:
 // the expression of the limiter's own apply, so the bits are those the
@@ -288,16 +299,16 @@ __device__ __forceinline__ void load_item_records(const int2 *jobs, const unsign
 // the loads: behind a branch, the waits for everything issued before would
 // have to assume either path and wait for the traces too.
 template <int NP, int EPB, bool LIM, class R, int NC>
-__device__ __forceinline__ void load_item_trace(const StageArgs<R> &A, int e0, FaceItem<R, NC> &it) {
+__device__ __forceinline__ void load_item_trace(const StageArgs<R> &A, int e0, FaceItem<R, NC> &it,
+                                                FaceMeans<LIM ? NC : 1> &fm) {
   const bool far = (unsigned)(it.job.y - e0) >= (unsigned)EPB;
   const size_t p = (size_t)(far ? it.job.y : e0);
   const R *g = A.q_in + (p * NP + (far ? it.pr & 255 : 0)) * NC;
 #pragma unroll
   for (int c = 0; c < NC; ++c) it.qp[c] = g[c];
   if constexpr (LIM) {
-    const double th = A.lim_th_in[p];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) it.qp[c] = lim_apply(it.qp[c], th, A.lim_mn_in[p * NC + c]);
+    for (int c = 0; c < NC; ++c) fm.m[c] = A.lim_mn_in[p * NC + c];
   }
 }
 
@@ -401,9 +412,11 @@ dg_stage_kernel(StageArgs<R> A) {
   __shared__ __align__(16) double sG[GEOM];
   const double *const sE = sG + 4 * max_face_geo(ND);
   __shared__ int sMap[NF * NFP];
-  // pending limiter factors of the tile's elements, then their means (q_in)
-  constexpr int NL = EPB * (NC + 1);
+  // limiter: the cell means of the tile's elements (q_in); the factors of
+  // the tile's elements, then of the elements behind its face jobs
+  constexpr int NL = EPB * NC;
   __shared__ double sLim[LIM ? NL : 1];
+  __shared__ double sTh[LIM ? EPB * (1 + NF) : 1];
   R *const sW = sB;
   R *const sS = sB + TILE;
 
@@ -437,7 +450,13 @@ dg_stage_kernel(StageArgs<R> A) {
   const int2 *const jobs = A.jobs + job0;
   const unsigned short *const ipr = A.ipr + NFP * job0;
   FaceItem<R, NC> it;
+  [[maybe_unused]] FaceMeans<LIM ? NC : 1> itm;
   load_item_records<NFP, MAXT>(jobs, ipr, tid < nitems ? tid : nitems - 1, it);
+  // limiter: thread i computes the factor of element i of the tile, then of
+  // the partner of face job i - EPB if that lies in another tile
+  const int thj = tid - EPB;
+  int2 thjob = int2{-1, 0};
+  if constexpr (LIM) thjob = jobs[thj < 0 ? 0 : thj < A.maxj ? thj : A.maxj - 1];
   const TileVec *const src = reinterpret_cast<const TileVec *>(A.q_in + tile0);
   TileVec tq[QPT];
 #pragma unroll
@@ -477,14 +496,11 @@ dg_stage_kernel(StageArgs<R> A) {
   }
   constexpr int LPT = (NL + S::BLOCK - 1) / S::BLOCK;
   double tl[LIM ? LPT : 1];
-  double tha = 1.0;
   if constexpr (LIM) {
 #pragma unroll
     for (int k = 0; k < LPT; ++k) {
       int t = k * S::BLOCK + tid;
-      t = t < NL ? t : NL - 1;
-      const double *g = t < EPB ? A.lim_th_in + e0 + t : A.lim_mn_in + (size_t)e0 * NC + (t - EPB);
-      tl[k] = *g;
+      tl[k] = A.lim_mn_in[(size_t)e0 * NC + (t < NL ? t : NL - 1)];
     }
   }
   const int nE = A.tile_count[tile];
@@ -497,7 +513,15 @@ dg_stage_kernel(StageArgs<R> A) {
   const double cdt = A.c * (A.inst_dt ? A.inst_dt[inst] : A.dt);
   const double post = A.inst_post ? A.inst_post[inst] : A.post_scale;
   if (!on) return;
-  load_item_trace<NP, EPB, LIM>(A, e0, it);
+  load_item_trace<NP, EPB, LIM>(A, e0, it, itm);
+  int the = e0, thnb[NF] = {0};
+  bool theta = false;
+  if constexpr (LIM) {
+    const bool far = thjob.x >= 0 && (unsigned)(thjob.y - e0) >= (unsigned)EPB && thj < A.maxj;
+    theta = thj < 0 || far;
+    the = thj < 0 ? e0 + tid : far ? thjob.y : e0;
+    bj_neighbours<NF>(the, A.conn, thnb);
+  }
   // FP64 form: the contraction streams the operator through the scalar
   // cache, which every launch starts with cold, a few rows at a time: a
   // chain of misses.  The launch's first blocks touch each line of a small
@@ -527,9 +551,9 @@ dg_stage_kernel(StageArgs<R> A) {
   const bool node = tid < nE * NP;
   if (LIM && !qa_is_in && tid < EPB * NP) {
     const size_t e = (size_t)e0 + nel;
-    tha = A.lim_th_a[e];
+    const double th = A.lim_th_a[e];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) qa_in[c] = lim_apply(qa_in[c], tha, A.lim_mn_a[e * NC + c]);
+    for (int c = 0; c < NC; ++c) qa_in[c] = lim_apply(qa_in[c], th, A.lim_mn_a[e * NC + c]);
   }
 #pragma unroll
   for (int k = 0; k < QPT; ++k) {
@@ -560,6 +584,17 @@ dg_stage_kernel(StageArgs<R> A) {
 #pragma unroll
     for (int k = 0; k < LPT; ++k)
       if (k * S::BLOCK + tid < NL) sLim[k * S::BLOCK + tid] = tl[k];
+    if (theta) {
+      const double th = bj_theta<NC, ND == 3, NF>(the, thnb, A.lim_mn_in, A.lim_ext_in, A.lim_eps2);
+      sTh[tid] = th;
+      if (thj < 0) A.lim_th_in[the] = th;
+    }
+    for (int i = tid + S::BLOCK; i < EPB + A.maxj; i += S::BLOCK) {  // more jobs than threads left
+      const int2 job = jobs[i - EPB];
+      if (job.x < 0 || (unsigned)(job.y - e0) < (unsigned)EPB) continue;
+      bj_neighbours<NF>(job.y, A.conn, thnb);
+      sTh[i] = bj_theta<NC, ND == 3, NF>(job.y, thnb, A.lim_mn_in, A.lim_ext_in, A.lim_eps2);
+    }
   }
   __syncthreads();
   // the q_in tile's pending limiter factors, applied in place to the
@@ -572,7 +607,7 @@ dg_stage_kernel(StageArgs<R> A) {
 #pragma unroll
         for (int v = 0; v < VW; ++v) {
           const int x = t * VW + v, el = x / (NP * NC), c = x % NC;
-          sW[x] = lim_apply(tq[k][v], sLim[el], sLim[EPB + el * NC + c]);
+          sW[x] = lim_apply(tq[k][v], sTh[el], sLim[el * NC + c]);
         }
       }
     }
@@ -595,7 +630,7 @@ dg_stage_kernel(StageArgs<R> A) {
   for (int t = tid; t < nitems; t += S::BLOCK) {
     if (t != tid) {
       load_item_records<NFP, MAXT>(jobs, ipr, t, it);
-      load_item_trace<NP, EPB, LIM>(A, e0, it);
+      load_item_trace<NP, EPB, LIM>(A, e0, it, itm);
     }
     if (it.job.x < 0) continue;
     const int el = it.job.x & 127, lf = (it.job.x >> 7) & 3, pin = (it.job.x >> 9) & 127;
@@ -607,6 +642,11 @@ dg_stage_kernel(StageArgs<R> A) {
     int other = __mul24(__mul24(pl, NP) + (int)(it.pr & 255), NC);
     if ((unsigned)pl >= (unsigned)EPB) {
       other = slot;
+      if constexpr (LIM) {
+        const double th = sTh[EPB + small_div<NFP, MAXT>(t)];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) it.qp[c] = lim_apply(it.qp[c], th, itm.m[c]);
+      }
 #pragma unroll
       for (int c = 0; c < NC; ++c) sB[slot + c] = it.qp[c];
     }
