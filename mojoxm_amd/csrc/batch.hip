@@ -42,6 +42,7 @@
 #include "diag.hpp"
 #include "limiter.hpp"
 #include "runtime.hpp"
+#include "transfer.hpp"
 
 namespace mxm {
 namespace {
@@ -315,6 +316,8 @@ struct Batch {
   std::map<int, std::unique_ptr<BInst>> insts;
   std::map<std::pair<int, int>, RefElem> refs;
   std::vector<std::unique_ptr<Staging>> staging;
+  HostPieces pieces;  // state transfers
+  int device = 0;     // the device current at create time
   int next_id = 0;
   // autotuned launch configuration per (group, grid-size octave)
   bool tune = true;
@@ -949,12 +952,9 @@ struct Batch {
 
   template <class R>
   void read_state(BGroup &g, DevBuf<R> (&q)[3], BInst &in, double *h) {
-    const size_t node = (size_t)g.NP * g.NC, tile_vals = (size_t)g.epb * node;
-    const size_t nv = (size_t)in.ntiles() * tile_vals;
-    std::vector<R> d(nv);
-    MXM_HIP(hipMemcpy(d.data(), q[0].p + (size_t)in.base_tile * tile_vals, nv * sizeof(R), hipMemcpyDeviceToHost));
-    for (int e = 0; e < in.K; ++e)
-      for (size_t c = 0; c < node; ++c) h[(size_t)e * node + c] = double(d[(size_t)in.t.til.dev_of[e] * node + c]);
+    const size_t node = (size_t)g.NP * g.NC;
+    MXM_HIP(move_state<true>(pieces, q[0].p + (size_t)in.base_tile * g.epb * node, in.t.til.ref_of.data(),
+                             in.ntiles() * g.epb, node, h, device, g.stream));
   }
 
   // the group of a placed instance, drained (placement first if needed)
@@ -1119,6 +1119,7 @@ int mxm_batch_create(int precision, void **out) {
     if (precision != MXM_PREC_FP64 && precision != MXM_PREC_FP32_MFMA) throw ArgError("unknown precision");
     auto b = std::make_unique<Batch>();
     b->prec = precision;
+    b->device = g_device;
     MXM_HIP(hipStreamCreateWithFlags(&b->cstream, hipStreamNonBlocking));
     *out = b.release();
     return MXM_OK;

@@ -19,6 +19,7 @@
 #include "host.hpp"
 #include "limiter.hpp"
 #include "runtime.hpp"
+#include "transfer.hpp"
 
 namespace mxm {
 namespace {
@@ -70,6 +71,7 @@ struct Solver {
   DevBuf<int2> jobs;
   DevBuf<unsigned short> ipr;
   int maxj = 0;
+  HostPieces pieces;  // state transfers
   // Device element order: tiles of lattice cells, each contiguous
   // (slot T*epb + el); the host side of the ABI keeps the reference order.
   Tiling til;
@@ -176,7 +178,7 @@ struct Solver {
     lmean.alloc((size_t)3 * Kd * NC);
     lext.alloc((size_t)3 * 2 * Kd * ncl());
     ltheta.alloc((size_t)3 * Kd);
-    clear_pending();
+    if (limiter) clear_pending();
     invJ.upload(t.invJ.data(), t.invJ.size());
     inv_vol.upload(t.inv_vol.data(), t.inv_vol.size());
     conn.upload(t.conn.data(), t.conn.size());
@@ -454,33 +456,17 @@ struct Solver {
   size_t state_elem_bytes() const { return prec == MXM_PREC_FP64 ? sizeof(double) : sizeof(float); }
   // q (reference order [K][NP][NC], FP64) <-> device slots and precision
   void upload_state(const double *h) {
-    const size_t node = (size_t)NP * NC, n = (size_t)Kd * node;
-    MXM_HIP(hipStreamSynchronize(stream));
-    if (prec == MXM_PREC_FP64) {
-      std::vector<double> d(n, 0.0);
-      for (int e = 0; e < K; ++e) std::memcpy(&d[(size_t)til.dev_of[e] * node], h + (size_t)e * node, node * sizeof(double));
-      MXM_HIP(hipMemcpy(q.p, d.data(), n * sizeof(double), hipMemcpyHostToDevice));
-    } else {
-      std::vector<float> d(n, 0.f);
-      for (int e = 0; e < K; ++e)
-        for (size_t k = 0; k < node; ++k) d[(size_t)til.dev_of[e] * node + k] = float(h[(size_t)e * node + k]);
-      MXM_HIP(hipMemcpy(f.p, d.data(), n * sizeof(float), hipMemcpyHostToDevice));
-    }
-    clear_pending();
+    if (prec == MXM_PREC_FP64)
+      MXM_HIP(move_state<false>(pieces, q.p, til.ref_of.data(), Kd, (size_t)NP * NC, h, device, stream));
+    else
+      MXM_HIP(move_state<false>(pieces, f.p, til.ref_of.data(), Kd, (size_t)NP * NC, h, device, stream));
+    if (limiter) clear_pending();  // nothing pending on a new state
   }
   void download_state(double *h) {
-    const size_t node = (size_t)NP * NC, n = (size_t)Kd * node;
-    MXM_HIP(hipStreamSynchronize(stream));
-    if (prec == MXM_PREC_FP64) {
-      std::vector<double> d(n);
-      MXM_HIP(hipMemcpy(d.data(), q.p, n * sizeof(double), hipMemcpyDeviceToHost));
-      for (int e = 0; e < K; ++e) std::memcpy(h + (size_t)e * node, &d[(size_t)til.dev_of[e] * node], node * sizeof(double));
-    } else {
-      std::vector<float> d(n);
-      MXM_HIP(hipMemcpy(d.data(), f.p, n * sizeof(float), hipMemcpyDeviceToHost));
-      for (int e = 0; e < K; ++e)
-        for (size_t k = 0; k < node; ++k) h[(size_t)e * node + k] = double(d[(size_t)til.dev_of[e] * node + k]);
-    }
+    if (prec == MXM_PREC_FP64)
+      MXM_HIP(move_state<true>(pieces, q.p, til.ref_of.data(), Kd, (size_t)NP * NC, h, device, stream));
+    else
+      MXM_HIP(move_state<true>(pieces, f.p, til.ref_of.data(), Kd, (size_t)NP * NC, h, device, stream));
   }
   size_t state_bytes() const { return q.bytes() + q1.bytes() + q2.bytes() + f.bytes() + f1.bytes() + f2.bytes(); }
   long long state_bytes_per_step() const { return 8LL * dof() * (long long)state_elem_bytes(); }
@@ -778,6 +764,7 @@ int mxm_dg_enable_limiter(void *h, int on, double eps) {
   return guarded([&] {
     Solver *s = as_solver(h);
     if (s->NC > kLimMaxNC) throw ArgError("limiter supports NC <= " + std::to_string(kLimMaxNC));
+    if (on && !s->limiter) s->clear_pending();  // between calls the stored state is what it is
     s->limiter = on != 0;
     s->eps = eps;
     return MXM_OK;
