@@ -64,7 +64,8 @@ struct Solver {
   // stage buffers (q, q1, q2)
   DevBuf<double> lmean, ltheta, lext;
   DevBuf<double> invJ, inv_vol, geom, Dt, Lt, w, dprm;
-  DevBuf<double> Dn, dpart, dout;  // diagnostics: nodal derivative, tile partials, results
+  DevBuf<double> Dn, dpart;  // diagnostics: nodal derivative, tile partials
+  PinBuf results;            // diagnostics and speed, written by the kernels
   DevBuf<float> Aop;
   DevBuf<int> conn;  // limiter: partner slot per face
   DevBuf<int> fmap, tile_count, tile_type;
@@ -87,6 +88,15 @@ struct Solver {
   // the same kernels, and one launch of many steps keeps the host out of
   // the way of short runs.
   static constexpr int kGraphSteps = 32;
+  // Calls of up to kDirectSteps steps launch their kernels on the stream: a
+  // graph launch costs more than the launches it replaces (16^2 Alfven wave,
+  // one step per call: 22.7 -> 18.8 us per step; from 3 steps on the graph is
+  // faster, 17.0).  So does the first call of up to kFirstSteps steps with a
+  // new dt, as in a loop that clamps to its frames or follows the CFL speed:
+  // capturing and uploading a graph to use it once took 44 us for one step
+  // and 29 per step for three, the launches take 18.7.
+  static constexpr int kDirectSteps = 2, kFirstSteps = 8;
+  double last_dt = 0.0;  // of the last call that launched directly
   StepGraph gfull;
   std::map<int, StepGraph> grem;
   double g_dt = 0.0, g_eps = 0.0;
@@ -378,11 +388,11 @@ struct Solver {
   void diagnostics(double *h) {
     const size_t per = (size_t)kDiagSums * 2 + kDiagMaxNC;
     if (dpart.n < (size_t)ntiles * per) dpart.alloc((size_t)ntiles * per);
-    if (dout.n < (size_t)(3 * NC + 2)) dout.alloc(3 * NC + 2);
+    results.reserve(3 * NC + 2);
     auto fill = [&](auto &a) {
       a.invJ = invJ.p, a.inv_vol = inv_vol.p, a.w = w.p, a.Dn = Dn.p, a.tile_count = tile_count.p;
       a.epb = til.epb, a.tile0 = 0, a.ntiles = ntiles, a.NC = NC, a.nvel = diag_nvel(phys);
-      a.part = dpart.p, a.pmax = dpart.p + (size_t)ntiles * kDiagSums * 2, a.out = dout.p;
+      a.part = dpart.p, a.pmax = dpart.p + (size_t)ntiles * kDiagSums * 2, a.out = results.p;
     };
     if (prec == MXM_PREC_FP64) {
       DiagArgs<double> a{};
@@ -395,8 +405,8 @@ struct Solver {
       fill(a);
       MXM_HIP(launch_diagnostics(dim, P, false, &a, stream));
     }
-    MXM_HIP(hipMemcpyAsync(h, dout.p, (3 * NC + 2) * sizeof(double), hipMemcpyDeviceToHost, stream));
     MXM_HIP(hipStreamSynchronize(stream));
+    std::memcpy(h, results.p, (3 * NC + 2) * sizeof(double));
     if (!diag_nvel(phys)) h[3 * NC] = h[3 * NC + 1] = std::nan("");
   }
 
@@ -424,18 +434,19 @@ struct Solver {
   // the largest signal speed over the nodes of the current state
   double max_wave_speed() {
     if (dpart.n < (size_t)ntiles) dpart.alloc(ntiles);
-    if (dout.n < 1) dout.alloc(1);
-    enqueue_max_speed(dpart.p, dout.p);
-    double h = 0.0;
-    MXM_HIP(hipMemcpyAsync(&h, dout.p, sizeof(double), hipMemcpyDeviceToHost, stream));
+    results.reserve(1);
+    enqueue_max_speed(dpart.p, results.p);
     MXM_HIP(hipStreamSynchronize(stream));
-    return h;
+    return results.p[0];
   }
+
+  // whether the graphs are those of the present settings and this dt
+  bool graphs_current(double dt) const { return dt == g_dt && limiter == g_lim && eps == g_eps && cfg == g_cfg; }
 
   // builds (if needed) the graphs that step(dt, n) replays
   void prepare(double dt, int n) {
     if (n <= 0) return;
-    if (dt != g_dt || limiter != g_lim || eps != g_eps || cfg != g_cfg) {
+    if (!graphs_current(dt)) {
       drop_graphs();
       g_dt = dt, g_lim = limiter, g_eps = eps, g_cfg = cfg;
     }
@@ -446,6 +457,13 @@ struct Solver {
 
   void step(double dt, int n) {
     if (n <= 0) return;
+    if (n <= kDirectSteps || (n <= kFirstSteps && !graphs_current(dt) && dt != last_dt)) {
+      last_dt = dt;
+      for (int k = 0; k < n; ++k)
+        for (int st = 0; st < 3; ++st) stage(st, dt);
+      if (limiter) materialize(0);
+      return;
+    }
     prepare(dt, n);
     for (; n >= kGraphSteps; n -= kGraphSteps) MXM_HIP(hipGraphLaunch(gfull.exec, stream));
     if (n) MXM_HIP(hipGraphLaunch(grem[n].exec, stream));
