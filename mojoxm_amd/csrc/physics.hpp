@@ -9,6 +9,7 @@
 //                             boundary_flux = numerical_flux(q, ghost(q))
 //   source(q, s)              pointwise source (kSource)
 //   limit(q)                  post-stage positivity fix (kLimit)
+//   kPost                     component damped after each step, -1 none
 // Trait physics (Advection, Euler) run in 3D and, with nz = 0, on
 // triangles; the 2D module physics (Euler2D, SW, GLM-MHD, Maxwell,
 // Advection2D) follow their reference kernels' inline physics.
@@ -61,6 +62,7 @@ template <class R>
 struct Advection {
   static constexpr int NC = 1;
   static constexpr bool kSource = false, kLimit = false;
+  static constexpr int kPost = -1;
   R v[3];
   R inflow;
   MXM_HD static Advection from(const double *p) { return {{R(p[0]), R(p[1]), R(p[2])}, R(p[3])}; }
@@ -91,6 +93,7 @@ template <class R, int FLUX, int EFIX = 0>
 struct Euler {
   static constexpr int NC = 5;
   static constexpr bool kSource = true, kLimit = true;
+  static constexpr int kPost = -1;
   static constexpr bool efix = EFIX != 0;
   R gamma, rmin_, pmin_;
   R g[3];
@@ -446,6 +449,7 @@ template <class R, int HLLC>
 struct Euler2D {
   static constexpr int NC = 4;
   static constexpr bool kSource = true, kLimit = false;
+  static constexpr int kPost = -1;
   R gamma, rmin_, pmin_, gx, gy;
   R inflow[4];
   MXM_HD static Euler2D from(const double *p) {
@@ -544,6 +548,7 @@ template <class R, int HLL>
 struct SW2D {
   static constexpr int NC = 3;
   static constexpr bool kSource = false, kLimit = false;
+  static constexpr int kPost = -1;
   R grav, hmin;
   R inflow[3];
   MXM_HD static SW2D from(const double *p) { return {R(p[0]), R(p[1]), {R(p[3]), R(p[4]), R(p[5])}}; }
@@ -609,6 +614,7 @@ template <class R>
 struct MHDGLM2D {
   static constexpr int NC = 7;
   static constexpr bool kSource = false, kLimit = false;
+  static constexpr int kPost = 6;  // psi, damped after each step
   R gamma, rmin_, pmin_, ch;
   R inflow[7];
   MXM_HD static MHDGLM2D from(const double *p) {
@@ -701,6 +707,7 @@ template <class R>
 struct Maxwell2D {
   static constexpr int NC = 6;
   static constexpr bool kSource = true, kLimit = false;
+  static constexpr int kPost = -1;
   R c, J[3], M[3], inflow[6];
   MXM_HD static Maxwell2D from(const double *p) {
     Maxwell2D m;
@@ -754,6 +761,7 @@ template <class R>
 struct Advection2D {
   static constexpr int NC = 1;
   static constexpr bool kSource = false, kLimit = false;
+  static constexpr int kPost = -1;
   R vx, vy, inflow;
   MXM_HD static Advection2D from(const double *p) { return {R(p[0]), R(p[1]), R(p[2])}; }
   template <int ND>
@@ -799,6 +807,7 @@ template <class R>
 struct ShallowWater3 {
   static constexpr int NC = 3;
   static constexpr bool kSource = false, kLimit = false;
+  static constexpr int kPost = -1;
   R g, hmin, inflow[3];
   MXM_HD static ShallowWater3 from(const double *p) {
     return {R(p[0]), R(p[1]), {R(p[2]), R(p[3]), R(p[4])}};
@@ -842,6 +851,7 @@ template <class R>
 struct Maxwell3 {
   static constexpr int NC = 6;
   static constexpr bool kSource = true, kLimit = false;
+  static constexpr int kPost = -1;
   R c, J[3], M[3], inflow[6];
   MXM_HD static Maxwell3 from(const double *p) {
     Maxwell3 m;
@@ -900,6 +910,7 @@ template <class R>
 struct IdealMHD3 {
   static constexpr int NC = 9;
   static constexpr bool kSource = true, kLimit = false;
+  static constexpr int kPost = -1;
   R gamma, rmin, pmin, ch, alpha, inflow[9];
   MXM_HD static IdealMHD3 from(const double *p) {
     IdealMHD3 m;
@@ -983,6 +994,7 @@ template <class R>
 struct TwoFluid3 {
   static constexpr int NC = 17;
   static constexpr bool kSource = true, kLimit = false;
+  static constexpr int kPost = -1;
   R ge, gi, qme, qmi, ieps0, cl, ch, alpha, rmin, pmin, inflow[17];
   MXM_HD static TwoFluid3 from(const double *p) {
     TwoFluid3 t;
