@@ -274,7 +274,7 @@ inline ElemTables build_elem_tables(const HostMesh &m, const RefElem &re, int nc
 // Reference operators in the layout of each arithmetic form.
 struct OpTables {
   std::vector<double> Dt, Lt;  // FP64: transposed, node columns zero-padded
-  std::vector<float> Aop;      // FP32-MFMA: [D_0 .. D_ND-1 | Lift], 16-row tiles
+  std::vector<float> Aop;      // FP32-MFMA: [D_0 .. D_ND-1 | Lift] in MFMA operand order (StageArgs::Aop)
 };
 
 inline OpTables build_operators(const RefElem &re, int dim, int NC, int prec) {
@@ -295,12 +295,14 @@ inline OpTables build_operators(const RefElem &re, int dim, int NC, int prec) {
     // columns: D_0 .. D_dim-1 (dim*NP, zero-padded to kvp), then Lift
     const int mt = mfma_mtiles(NP), kp = mfma_kpad(dim, NP, NFP), kvp = mfma_kvpad(dim, NP);
     o.Aop.assign((size_t)mt * 16 * kp, 0.f);
+    auto put = [&](int i, int k, double v) {
+      o.Aop[((size_t)(k / 4) * mt + i / 16) * 64 + (k % 4) * 16 + i % 16] = float(v);
+    };
     for (int i = 0; i < NP; ++i) {
       for (int d = 0; d < dim; ++d)
-        for (int j = 0; j < NP; ++j) o.Aop[(size_t)i * kp + d * NP + j] = float(re.D[((size_t)d * NP + i) * NP + j]);
+        for (int j = 0; j < NP; ++j) put(i, d * NP + j, re.D[((size_t)d * NP + i) * NP + j]);
       for (int fc = 0; fc < NF; ++fc)
-        for (int r = 0; r < NFP; ++r)
-          o.Aop[(size_t)i * kp + kvp + fc * NFP + r] = float(re.Lift[((size_t)fc * NP + i) * NFP + r]);
+        for (int r = 0; r < NFP; ++r) put(i, kvp + fc * NFP + r, re.Lift[((size_t)fc * NP + i) * NFP + r]);
     }
   }
   return o;

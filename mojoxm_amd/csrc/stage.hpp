@@ -93,7 +93,8 @@ struct StageArgs {
   const int *tile_type;   // [ntiles] cell element of the tile's first slot
   const double *Dt;       // FP64 form: [ND*NP (k,j)][NPAD (i)] transposed D_ref, zero padded
   const double *Lt;       // FP64 form: [NF*NFP (f,r)][NPAD (i)] transposed Lift_ref, zero padded
-  const float *Aop;       // FP32 form: [16*MT (i)][KPAD (k)] = [D_0 .. D_ND-1 | Lift], zero padded
+  const float *Aop;       // FP32 form: [D_0 .. D_ND-1 | Lift], zero padded, in the order the MFMA operand reads it:
+                          // [KPAD/4][MT][lane 16 g + r] = row 16 m + r, column 4 k + g
   const int *fmap;        // [NF][NFP] element node of each reference face slot
   const int2 *jobs;       // [ntiles*maxj] {el | lf<<7 | pin<<9 | plf<<16 | side<<18 | bc<<19 | geometry<<22
                           //  (-1: padding), partner slot}
@@ -388,20 +389,11 @@ dg_stage_kernel(StageArgs<R> A) {
   constexpr int NB0 = stage_operand_len(kMFMA, TILE, NCOLS, KV, KVP, NFF, KPAD, NT * 16);
   constexpr int QA0 = (NB0 + 3) / 4 * 4;  // past every operand read and the zeroed padding, 16-byte aligned
   constexpr int NB = kQaLds ? QA0 + TILE : NB0;
-  // FP32-MFMA: the operator [D | Lift] staged in LDS when it is at most
-  // 16 KB (2D, 3D P <= 3), else read from global memory (L2) in the loop
-  constexpr int NA = kMFMA ? MT * 16 * KPAD : 0;
-  constexpr bool kStageA = kMFMA && NA * 4 <= 16384;
-  // LDS row stride of the staged operator: 4 mod 8 words, so the 16 rows
-  // x 4 columns an A operand read touches fall in 64 distinct banks (a
-  // stride of 32, as 2D P = 3 has, put all 16 rows in one bank group)
-  constexpr int KAS = KPAD % 8 == 4 ? KPAD : KPAD + 4;
   // sW = sB: first the q_in tile as [el][j][c] (TILE contiguous values);
   // after the lift product the contravariant nodal fluxes as [k][j][el][c]
   // (row kj at kj*NCOLS); after the volume product the result as
   // [el][i][c].  sS = sB + TILE: face fluxes [f*NFP + r][el][c].
   __shared__ __align__(16) R sB[NB];
-  __shared__ float sA[kStageA ? MT * 16 * KAS : 1];
   // the geometry (StageArgs::geom): face normals and areas, then invJ and
   // inv_vol of each element of a lattice cell.  A lattice has a handful of
   // each, so a tile reads 0.2 to 1 KB for them, the same for every tile,
@@ -486,15 +478,6 @@ dg_stage_kernel(StageArgs<R> A) {
     }
   }
   const int fm = A.fmap[tid < NFF ? tid : NFF - 1];
-  constexpr int APT = kStageA ? (NA + S::BLOCK - 1) / S::BLOCK : 0;
-  float ta[APT > 0 ? APT : 1];
-  if constexpr (kStageA) {
-#pragma unroll
-    for (int k = 0; k < APT; ++k) {
-      const int t = k * S::BLOCK + tid;
-      ta[k] = A.Aop[(k + 1) * S::BLOCK <= NA || t < NA ? t : NA - 1];
-    }
-  }
   constexpr int LPT = (NL + S::BLOCK - 1) / S::BLOCK;
   double tl[LIM ? LPT : 1];
   if constexpr (LIM) {
@@ -570,13 +553,6 @@ dg_stage_kernel(StageArgs<R> A) {
         const int t = k * S::BLOCK + tid;
         if ((k + 1) * S::BLOCK <= TV || t < TV) reinterpret_cast<TileVec *>(sB + QA0)[t] = tqa[k];
       }
-    }
-  }
-  if constexpr (kStageA) {
-#pragma unroll
-    for (int k = 0; k < APT; ++k) {
-      const int t = k * S::BLOCK + tid, row = t / KPAD;
-      if (t < NA) sA[row * KAS + t - row * KPAD] = ta[k];
     }
   }
   if constexpr (kMFMA)
@@ -733,6 +709,23 @@ dg_stage_kernel(StageArgs<R> A) {
       }
     }
   }
+  // FP32-MFMA: the operator entries of a whole product go straight to the
+  // registers of the lanes that feed them to the MFMA, one coalesced load
+  // each, ahead of the barrier before the product.  Staged in LDS, the
+  // operator took 12.8 of the 28.7 KB of a 3D P = 3 block and held it to 5
+  // blocks per CU (us per stage: 32^3 Taylor-Green 115 -> 108, 19^3 30.7 ->
+  // 29.3, 113^2 P = 4 Maxwell 11.3 -> 11.0, 128^2 vortex 8.8 -> 8.6).
+  constexpr int KL = (KPAD - KVP) / 4, KD = KVP / 4;      // k-steps of the lift and volume products
+  constexpr bool kAhead = kMFMA && MT * (KL > KD ? KL : KD) <= 32;
+  const int l = tid & 63, lr = l & 15, lg = l >> 4;
+  auto aop = [&](int k, int m) { return A.Aop[(k * MT + m) * 64 + l]; };
+  [[maybe_unused]] float al[kAhead ? KL : 1][MT], ad[kAhead ? KD : 1][MT];
+  if constexpr (kAhead) {
+#pragma unroll
+    for (int k = 0; k < KL; ++k)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) al[k][m] = aop(KD + k, m);
+  }
   __syncthreads();
 
   // ---- 3. contractions ----------------------------------------------------
@@ -748,7 +741,6 @@ dg_stage_kernel(StageArgs<R> A) {
   // 4 g + v (v < 4), column col0 + r.
   constexpr int NTW = (NT + S::BLOCK / 64 - 1) / (S::BLOCK / 64);  // column tiles per wave
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l = tid & 63, lr = l & 15, lg = l >> 4;
   mxm_float4 macc[kMFMA ? MT : 1][kMFMA ? NTW : 1];
   // FP64 on the VALU: the (element, component) columns are the lanes;
   // each wave group produces IH consecutive output nodes, so the operator
@@ -822,8 +814,8 @@ dg_stage_kernel(StageArgs<R> A) {
       use(0, last);
     }
   };
-  // One 4-deep step of the MFMA product over operator columns k0.. and
-  // operand rows kb.. of Bb.  Branch-free, so that the operand reads of many
+  // One 4-deep step of the MFMA product: operator entries a, operand rows
+  // 4 kb .. of Bb.  Branch-free, so that the operand reads of many
   // steps are in flight together: a wave's column tile past the last one
   // repeats the last (its result is not stored).  With a branch around it
   // each step waited for its own LDS reads (us per stage: 128^2 vortex 9.4 ->
@@ -834,20 +826,23 @@ dg_stage_kernel(StageArgs<R> A) {
     const int nt = wave * NTW + w;
     bcol[w] = lg * NCOLS + (nt < NT ? nt : NT - 1) * 16 + lr;
   }
-  auto kstep = [&](const R *Bb, int k0, int kb) {
-    float a[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      if constexpr (kStageA)
-        a[m] = sA[(m * 16 + lr) * KAS + k0 + lg];
-      else
-        a[m] = A.Aop[(m * 16 + lr) * KPAD + k0 + lg];
-    }
+  auto kstep = [&](const R *Bb, const float (&a)[MT], int kb) {
 #pragma unroll
     for (int w = 0; w < NTW; ++w) {
-      const float bv = float(Bb[kb * NCOLS + bcol[w]]);
+      const float bv = float(Bb[kb * 4 * NCOLS + bcol[w]]);
 #pragma unroll
       for (int m = 0; m < MT; ++m) macc[m][w] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m], bv, macc[m][w], 0, 0, 0);
+    }
+  };
+  // the product over the k-steps [k0, k1) of the operator, entries loaded as
+  // it goes
+  [[maybe_unused]] auto product = [&](const R *Bb, int k0, int k1) {
+#pragma unroll 4
+    for (int k = k0; k < k1; ++k) {
+      float a[MT];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) a[m] = aop(k, m);
+      kstep(Bb, a, k - k0);
     }
   };
 
@@ -857,12 +852,11 @@ dg_stage_kernel(StageArgs<R> A) {
     for (int m = 0; m < MT; ++m)
 #pragma unroll
       for (int w = 0; w < NTW; ++w) macc[m][w] = mxm_float4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (kStageA) {
+    if constexpr (kAhead) {
 #pragma unroll
-      for (int k0 = KVP; k0 < KPAD; k0 += 4) kstep(sS, k0, k0 - KVP);
+      for (int k = 0; k < KL; ++k) kstep(sS, al[k], k);
     } else {
-#pragma unroll 4
-      for (int k0 = KVP; k0 < KPAD; k0 += 4) kstep(sS, k0, k0 - KVP);
+      product(sS, KD, KD + KL);
     }
   } else {
 #pragma unroll
@@ -891,16 +885,21 @@ dg_stage_kernel(StageArgs<R> A) {
   }
   if constexpr (kMFMA && KVP > KV)
     for (int t = KV * NCOLS + tid; t < KVP * NCOLS; t += S::BLOCK) sB[t] = R(0);
+  if constexpr (kAhead) {
+#pragma unroll
+    for (int k = 0; k < KD; ++k)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) ad[k][m] = aop(k, m);
+  }
   __syncthreads();
 
   // ---- 3c. volume product, result as [el][i][c] ---------------------------
   if constexpr (kMFMA) {
-    if constexpr (kStageA) {
+    if constexpr (kAhead) {
 #pragma unroll
-      for (int k0 = 0; k0 < KVP; k0 += 4) kstep(sW, k0, k0);
+      for (int k = 0; k < KD; ++k) kstep(sW, ad[k], k);
     } else {
-#pragma unroll 4
-      for (int k0 = 0; k0 < KVP; k0 += 4) kstep(sW, k0, k0);
+      product(sW, 0, KD);
     }
     __syncthreads();
 #pragma unroll
