@@ -375,25 +375,22 @@ dg_stage_kernel(StageArgs<R> A) {
   constexpr int KPAD = kMFMA ? mfma_kpad(ND, NP, NFP) : KV + NFF;
   constexpr int MT = mfma_mtiles(NP);
   constexpr int NT = (NCOL + 15) / 16;
-  // 2D kernels without the limiter, FP32 form with 7 or more components
-  // (GLM-MHD) and FP64 form with at most 5: q_a is loaded with the tile
-  // into LDS past the operand array and read by the node threads in 2b,
-  // instead of waiting in NC registers through the face phase, the
-  // register peak.  FP32 GLM-MHD then fits 6 waves per SIMD without spills
-  // (its 384^2 stage 2 % faster) and the FP64 Euler kernels 5 (96 VGPRs,
-  // 31.8 KB LDS: the 512^2 vortex stage 4 % faster, C2 0.5 %).  The FP32
-  // Euler kernels lost 1 % (their registers were not the limit), FP64
-  // GLM-MHD and Maxwell would become LDS-bound, and the 3D kernels' LDS
-  // would bound their blocks per CU.
-  constexpr bool kQaLds = !LIM && ND == 2 && (kMFMA ? NC >= 7 : NC <= 5);
+  // q_a is loaded by the node threads where they use it (2b), not with the
+  // tile: held through the face phase, the register peak, it costs NC
+  // registers (or as much LDS as the tile), and other blocks cover the wait.
+  // The FP64 Euler kernel on triangles goes from 30.7 to 21 KB of LDS and
+  // from 82 to 80 VGPRs, 5 to 6 waves per SIMD (us per stage: 128^2 vortex
+  // 13.6 -> 13.1, 512^2 144 -> 138; 384^2 GLM-MHD FP64 110 -> 104, FP32 61.1
+  // -> 59.6; limited 192^2 Sod FP64 32.5 -> 29.8).  The FP32 kernels of at
+  // most 5 components fit 8 waves either way and keep the early load (512^2
+  // vortex 81.5, late 83.3).
+  constexpr bool kQaLate = !kMFMA || NC >= 6 || LIM;
   constexpr int NB0 = stage_operand_len(kMFMA, TILE, NCOLS, KV, KVP, NFF, KPAD, NT * 16);
-  constexpr int QA0 = (NB0 + 3) / 4 * 4;  // past every operand read and the zeroed padding, 16-byte aligned
-  constexpr int NB = kQaLds ? QA0 + TILE : NB0;
   // sW = sB: first the q_in tile as [el][j][c] (TILE contiguous values);
   // after the lift product the contravariant nodal fluxes as [k][j][el][c]
   // (row kj at kj*NCOLS); after the volume product the result as
   // [el][i][c].  sS = sB + TILE: face fluxes [f*NFP + r][el][c].
-  __shared__ __align__(16) R sB[NB];
+  __shared__ __align__(16) R sB[NB0];
   // the geometry (StageArgs::geom): face normals and areas, then invJ and
   // inv_vol of each element of a lattice cell.  A lattice has a handful of
   // each, so a tile reads 0.2 to 1 KB for them, the same for every tile,
@@ -457,25 +454,17 @@ dg_stage_kernel(StageArgs<R> A) {
     const int t = k * S::BLOCK + tid;
     tq[k] = src[(k + 1) * S::BLOCK <= TV || t < TV ? t : TV - 1];
   }
-  // q_a (through LDS to 2b when kQaLds, else of the own node and in the
-  // state precision until 2b); when q_a is the stage input (SSPRK3 stage 1)
-  // it is read from the LDS copy of the tile
+  // q_a of the own node, in the state precision until 2b; when q_a is the
+  // stage input (SSPRK3 stage 1) it is read from the LDS copy of the tile
   const bool qa_is_in = A.q_a == A.q_in;
-  TileVec tqa[kQaLds ? QPT : 1];
   R qa_in[NC];
-  if (!qa_is_in) {
-    if constexpr (kQaLds) {
-      const TileVec *const sa = reinterpret_cast<const TileVec *>(A.q_a + tile0);
+  auto load_qa = [&] {
+    const R *g = A.q_a + tile0 + (tid < EPB * NP ? tid : EPB * NP - 1) * NC;
 #pragma unroll
-      for (int k = 0; k < QPT; ++k) {
-        const int t = k * S::BLOCK + tid;
-        tqa[k] = sa[(k + 1) * S::BLOCK <= TV || t < TV ? t : TV - 1];
-      }
-    } else {
-      const R *g = A.q_a + tile0 + (tid < EPB * NP ? tid : EPB * NP - 1) * NC;
-#pragma unroll
-      for (int c = 0; c < NC; ++c) qa_in[c] = g[c];
-    }
+    for (int c = 0; c < NC; ++c) qa_in[c] = g[c];
+  };
+  if constexpr (!kQaLate) {
+    if (!qa_is_in) load_qa();
   }
   const int fm = A.fmap[tid < NFF ? tid : NFF - 1];
   constexpr int LPT = (NL + S::BLOCK - 1) / S::BLOCK;
@@ -533,12 +522,15 @@ dg_stage_kernel(StageArgs<R> A) {
   // thread tid owns output node (el, i) = (tid / NP, tid % NP): EPB*NP <= BLOCK
   const int nel = small_div<NP, S::BLOCK>(tid), nod = tid - nel * NP;
   const bool node = tid < nE * NP;
-  if (LIM && !qa_is_in && tid < EPB * NP) {
-    const size_t e = (size_t)e0 + nel;
-    const double th = A.lim_th_a[e];
+  auto limit_qa = [&] {
+    if (LIM && !qa_is_in && tid < EPB * NP) {
+      const size_t e = (size_t)e0 + nel;
+      const double th = A.lim_th_a[e];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) qa_in[c] = lim_apply(qa_in[c], th, A.lim_mn_a[e * NC + c]);
-  }
+      for (int c = 0; c < NC; ++c) qa_in[c] = lim_apply(qa_in[c], th, A.lim_mn_a[e * NC + c]);
+    }
+  };
+  if constexpr (!kQaLate) limit_qa();
 #pragma unroll
   for (int k = 0; k < QPT; ++k) {
     const int t = k * S::BLOCK + tid;
@@ -546,15 +538,6 @@ dg_stage_kernel(StageArgs<R> A) {
   }
   if (tid < GEOM) sG[tid] = tg;
   if (tid < NFF) sMap[tid] = fm;
-  if constexpr (kQaLds) {
-    if (!qa_is_in) {
-#pragma unroll
-      for (int k = 0; k < QPT; ++k) {
-        const int t = k * S::BLOCK + tid;
-        if ((k + 1) * S::BLOCK <= TV || t < TV) reinterpret_cast<TileVec *>(sB + QA0)[t] = tqa[k];
-      }
-    }
-  }
   if constexpr (kMFMA)
     for (int t = TILE + NFF * NCOLS + tid; t < NB0; t += S::BLOCK) sB[t] = R(0);
   if constexpr (LIM) {
@@ -661,6 +644,12 @@ dg_stage_kernel(StageArgs<R> A) {
   // read of the q_in tile is done.
   R Fk[ND * NC];
   double qa[NC];
+  if constexpr (kQaLate) {
+    if (!qa_is_in) {
+      load_qa();
+      limit_qa();
+    }
+  }
   if (node) {
     const R *q = &sQ[tid * NC];
     R F[ND * NC];
@@ -691,12 +680,6 @@ dg_stage_kernel(StageArgs<R> A) {
           for (int d = 0; d < ND; ++d) v += iJ[k * ND + d] * double(F[d * NC + c]);
           Fk[k * NC + c] = R(v);
         }
-    }
-    if constexpr (kQaLds) {
-      if (!qa_is_in) {
-#pragma unroll
-        for (int c = 0; c < NC; ++c) qa_in[c] = sB[QA0 + tid * NC + c];
-      }
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) qa[c] = A.a * double(qa_is_in ? q[c] : qa_in[c]) + A.b * double(q[c]);
