@@ -420,7 +420,7 @@ struct Batch {
     in->K = m.K, in->NP = m.NP;
     if (!q0 || n != (long long)m.K * m.NP * nc) throw ArgError("initial state length must be K*NP*NC");
     in->q0.assign(q0, q0 + n);
-    in->t = build_elem_tables(m, re, nc, false);
+    in->t = build_elem_tables(m, re, nc, false, prec == MXM_PREC_FP32_MFMA);
     in->id = next_id++;
     BGroup &g = group_of_key(*in);
     g.waiting.push_back(in->id);
@@ -654,7 +654,7 @@ struct Batch {
     else
       state_trio(na.qf, g.ar.qf);
     std::vector<double> ij(slots * dd, 0.0), iv(slots, 0.0);
-    const size_t gl = stage_geom_len(g.dim);
+    const size_t gl = stage_geom_len(g.dim, g.prec == MXM_PREC_FP32_MFMA);
     std::vector<double> geo(cap_slots * gl, 0.0);
     std::vector<int> cn(slots * NF);
     std::vector<int2> jb((size_t)cap_tiles * maxj);
@@ -1099,7 +1099,7 @@ int footprint(int dim, const void *desc, int P, int phys, int prec, int limiter,
     check_bc(d->bc, 4);
     m = build_mesh_2d(d->nx, d->ny, d->lx, d->ly, d->bc, P, re);
   }
-  ElemTables t = build_elem_tables(m, re, nc, false);
+  ElemTables t = build_elem_tables(m, re, nc, false, prec == MXM_PREC_FP32_MFMA);
   *out = (long long)instance_bytes(t, m.NP, nc, m.NFP, dim, prec, limiter != 0);
   return MXM_OK;
 }

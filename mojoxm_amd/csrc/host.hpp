@@ -82,6 +82,12 @@ Tiling build_tiling(const HostMesh &m, int epb, int NFP);
 constexpr int max_face_geo(int dim) { return dim == 3 ? 18 : 5; }
 // Elements of a lattice cell
 constexpr int cell_elems(int dim) { return dim == 3 ? 6 : 2; }
+// Length of the stage kernel's geometry table (StageArgs::geom), and of an
+// element's part of it
+constexpr int stage_geom_elem(int dim, bool fp32) { return dim * dim + (fp32 ? max_face_geo(dim) : 1); }
+constexpr int stage_geom_len(int dim, bool fp32) {
+  return 4 * max_face_geo(dim) + cell_elems(dim) * stage_geom_elem(dim, fp32);
+}
 
 // Face-flux work lists of the stage kernel.  Within a tile, a face whose
 // two sides both lie in the tile is evaluated once (by its side-0

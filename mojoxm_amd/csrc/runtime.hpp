@@ -224,13 +224,14 @@ struct ElemTables {
   std::vector<double> invJ, inv_vol;
   std::vector<int> conn;  // limiter neighbours: the partner slot of each face (its own slot on a boundary)
   // the stage kernel's geometry (StageArgs::geom): the distinct face normals
-  // and areas, then invJ and inv_vol of each element of a lattice cell
+  // and areas, then invJ and inv_vol (FP32 form: -inv_vol times each area) of
+  // each element of a lattice cell
   std::vector<double> geom;
   std::vector<int> tile_type;  // cell element of each tile's first slot
 };
 
 // wide: tiles of the wide tile size (stage_epb)
-inline ElemTables build_elem_tables(const HostMesh &m, const RefElem &re, int nc, bool wide) {
+inline ElemTables build_elem_tables(const HostMesh &m, const RefElem &re, int nc, bool wide, bool fp32) {
   ElemTables t;
   Connectivity cn = build_connectivity(m, re);
   t.til = build_tiling(m, stage_epb(m.dim, m.NP, m.NFP, nc, wide), m.NFP);
@@ -255,7 +256,8 @@ inline ElemTables build_elem_tables(const HostMesh &m, const RefElem &re, int nc
   const int epc = cell_elems(m.dim);
   for (int y = 0; y < epc; ++y) {
     t.geom.insert(t.geom.end(), &m.elem_invJ[(size_t)y * dd], &m.elem_invJ[(size_t)y * dd] + dd);
-    t.geom.push_back(m.elem_inv_vol[y]);
+    if (!fp32) t.geom.push_back(m.elem_inv_vol[y]);
+    for (int g = 0; fp32 && g < max_face_geo(m.dim); ++g) t.geom.push_back(-m.elem_inv_vol[y] * t.geom[4 * g + 3]);
   }
   // every element has the geometry of its place in its cell, and a tile's
   // slots run through those places in order

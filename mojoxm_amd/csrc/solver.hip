@@ -169,7 +169,7 @@ struct Solver {
   // with a zero state and nothing pending; graphs are dropped
   void layout(const HostMesh &m, const RefElem &re) {
     drop_graphs();
-    ElemTables t = build_elem_tables(m, re, NC, wide);
+    ElemTables t = build_elem_tables(m, re, NC, wide, prec == MXM_PREC_FP32_MFMA);
     til = std::move(t.til);
     Kd = til.slots();
     ntiles = til.ntiles;

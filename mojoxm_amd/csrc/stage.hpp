@@ -32,11 +32,10 @@
 //   R = float   FP32-MFMA: FP32 state, fluxes and traces; the volume and
 //               LIFT contractions are one [D | Lift] x [F ; S] product per
 //               tile on V_MFMA_F32_16X16X4F32 with FP32 accumulation, the
-//               surface fluxes pre-scaled by -inv_vol s area; geometry and
-//               Jacobians are stored in FP64 (the nodal flux is mapped by
-//               invJ rounded to FP32), and the RK combine and the
-//               positivity rescue are FP64; the stored state is rounded
-//               stochastically.
+//               surface fluxes pre-scaled by -inv_vol s area; geometry is
+//               formed in FP64 and rounded once to FP32, and the RK combine
+//               and the positivity rescue are FP64; the stored state is
+//               rounded stochastically.
 // Blocks are mapped to tiles so that each of the 8 XCDs walks a contiguous
 // range of tiles: face neighbours then mostly hit the XCD's own L2.
 #pragma once
@@ -89,7 +88,8 @@ struct StageArgs {
   const int *tile_count;  // [ntiles] elements in each tile (slots T*EPB ..)
   const double *geom;     // [n_inst][stage_geom_len]: the mesh's distinct face normals and areas
                           // ([max_face_geo][4]), then per element of a lattice cell invJ (ND*ND, rows =
-                          // reference directions) and inv_vol (1/(6V) or 1/(2A))
+                          // reference directions) and inv_vol (1/(6V) or 1/(2A)), in the FP32 form
+                          // -inv_vol times each of those areas
   const int *tile_type;   // [ntiles] cell element of the tile's first slot
   const double *Dt;       // FP64 form: [ND*NP (k,j)][NPAD (i)] transposed D_ref, zero padded
   const double *Lt;       // FP64 form: [NF*NFP (f,r)][NPAD (i)] transposed Lift_ref, zero padded
@@ -163,7 +163,6 @@ constexpr int stage_lds_bytes(int ND, int NP, int NFP, int NC, int epb) {
               : ND * NP * (epb * NC + 1)) * 8 +
          epb * (ND * ND + 1) * 8 + (ND + 1) * NFP * 4;
 }
-constexpr int stage_geom_len(int ND) { return 4 * max_face_geo(ND) + cell_elems(ND) * (ND * ND + 1); }
 constexpr int stage_epb(int ND, int NP, int NFP, int NC, bool wide = false) {
   const int cell = ND == 3 ? 6 : 2;
   int e = 256 / NP;
@@ -397,10 +396,14 @@ dg_stage_kernel(StageArgs<R> A) {
   // where a record per face and per slot took 3 KB: 77 of the 251 MB that
   // the FP32 512^2 vortex stage fetched (90.6 -> 86.0 us; 32^3 Taylor-Green
   // FP64 186 -> 181, 16^3 P = 2 advection 7.9 -> 7.5).
-  constexpr int EPC = cell_elems(ND), GEL = ND * ND + 1, GEOM = stage_geom_len(ND);
+  // The FP32 form keeps its table in FP32 with the face scales multiplied
+  // out, as it uses them: one read per face item where an FP64 product and
+  // conversions stood (32^3 Taylor-Green 108.6 -> 107.0, 384^2 GLM-MHD 60.7
+  // -> 59.8, 128^2 vortex 8.67 -> 8.57).
+  constexpr int EPC = cell_elems(ND), GEL = stage_geom_elem(ND, kMFMA), GEOM = stage_geom_len(ND, kMFMA);
   static_assert(GEOM <= 256, "one geometry value per thread");
-  __shared__ __align__(16) double sG[GEOM];
-  const double *const sE = sG + 4 * max_face_geo(ND);
+  __shared__ __align__(16) R sG[GEOM];
+  const R *const sE = sG + 4 * max_face_geo(ND);
   __shared__ int sMap[NF * NFP];
   // limiter: the cell means of the tile's elements (q_in); the factors of
   // the tile's elements, then of the elements behind its face jobs
@@ -536,7 +539,7 @@ dg_stage_kernel(StageArgs<R> A) {
     const int t = k * S::BLOCK + tid;
     if ((k + 1) * S::BLOCK <= TV || t < TV) reinterpret_cast<TileVec *>(sW)[t] = tq[k];
   }
-  if (tid < GEOM) sG[tid] = tg;
+  if (tid < GEOM) sG[tid] = R(tg);
   if (tid < NFF) sMap[tid] = fm;
   if constexpr (kMFMA)
     for (int t = TILE + NFF * NCOLS + tid; t < NB0; t += S::BLOCK) sB[t] = R(0);
@@ -595,7 +598,8 @@ dg_stage_kernel(StageArgs<R> A) {
     if (it.job.x < 0) continue;
     const int el = it.job.x & 127, lf = (it.job.x >> 7) & 3, pin = (it.job.x >> 9) & 127;
     const int bc = (it.job.x >> 19) & 7;
-    const double *const geo = sG + 4 * (it.job.x >> 22);  // normal, area
+    const int gi = it.job.x >> 22;
+    const R *const geo = sG + 4 * gi;  // normal, area
     const int fr = lf * NFP + (t - small_div<NFP, MAXT>(t) * NFP);
     const int pl = it.job.y - e0, slot = TILE + fr * NCOLS + el * NC;
     const int mine = (el * NP + sMap[fr]) * NC;
@@ -613,7 +617,7 @@ dg_stage_kernel(StageArgs<R> A) {
     // left = side-0 trace; right = side-1 trace or the ghost of the left
     const bool s0 = !(it.job.x & (1 << 18));
     const R *const pL = sB + (s0 ? mine : other), *const pR = sB + (s0 ? other : mine);
-    const R n[3] = {R(geo[0]), R(geo[1]), ND == 3 ? R(geo[2]) : R(0)};
+    const R n[3] = {geo[0], geo[1], ND == 3 ? geo[2] : R(0)};
     R ql[NC], qr[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) ql[c] = pL[c];
@@ -624,15 +628,15 @@ dg_stage_kernel(StageArgs<R> A) {
       for (int c = 0; c < NC; ++c) qr[c] = pR[c];
     R Fs[NC];
     phys.template numerical_flux<ND>(ql, qr, n, Fs);
-    const double sa = s0 ? geo[3] : -geo[3];
     // FP64 form: s area F*, lifted and scaled by -inv_vol in the
     // contraction; FP32 form: -inv_vol s area F*, ready for the product
-    const R own = kMFMA ? R(-sE[cell_type(el) * GEL + ND * ND] * sa) : R(sa);
+    const R w = kMFMA ? sE[cell_type(el) * GEL + ND * ND + gi] : geo[3], own = s0 ? w : -w;
 #pragma unroll
     for (int c = 0; c < NC; ++c) sB[slot + c] = own * Fs[c];
     if (pin) {
       const int plf = (it.job.x >> 16) & 3, rs = it.pr >> 8;
-      const R oth = kMFMA ? R(sE[cell_type(pin - 1) * GEL + ND * ND] * sa) : R(-sa);
+      // (a paired job is its side-0 element's)
+      const R oth = kMFMA ? -sE[cell_type(pin - 1) * GEL + ND * ND + gi] : -own;
 #pragma unroll
       for (int c = 0; c < NC; ++c) sS[(plf * NFP + rs) * NCOLS + (pin - 1) * NC + c] = oth * Fs[c];
     }
@@ -654,20 +658,17 @@ dg_stage_kernel(StageArgs<R> A) {
     const R *q = &sQ[tid * NC];
     R F[ND * NC];
     phys.template flux<ND>(q, F);
-    const double *iJ = sE + cell_type(nel) * GEL;
+    const R *iJ = sE + cell_type(nel) * GEL;
     if constexpr (kMFMA) {
-      // FP32 form: the mapping in FP32 (invJ rounded once per node), as
+      // FP32 form: the mapping in FP32 (invJ rounded to FP32), as
       // the volume product that takes its result is
-      float jf[ND * ND];
-#pragma unroll
-      for (int t = 0; t < ND * ND; ++t) jf[t] = float(iJ[t]);
 #pragma unroll
       for (int k = 0; k < ND; ++k)
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
           float v = 0.f;
 #pragma unroll
-          for (int d = 0; d < ND; ++d) v += jf[k * ND + d] * F[d * NC + c];
+          for (int d = 0; d < ND; ++d) v += iJ[k * ND + d] * F[d * NC + c];
           Fk[k * NC + c] = v;
         }
     } else {
