@@ -420,7 +420,7 @@ struct Batch {
     in->K = m.K, in->NP = m.NP;
     if (!q0 || n != (long long)m.K * m.NP * nc) throw ArgError("initial state length must be K*NP*NC");
     in->q0.assign(q0, q0 + n);
-    in->t = build_elem_tables(m, re, nc, false, prec == MXM_PREC_FP32_MFMA);
+    in->t = build_elem_tables(m, re, nc, false, prec == MXM_PREC_FP32_MFMA, kRoomBatch);
     in->id = next_id++;
     BGroup &g = group_of_key(*in);
     g.waiting.push_back(in->id);
@@ -1099,7 +1099,7 @@ int footprint(int dim, const void *desc, int P, int phys, int prec, int limiter,
     check_bc(d->bc, 4);
     m = build_mesh_2d(d->nx, d->ny, d->lx, d->ly, d->bc, P, re);
   }
-  ElemTables t = build_elem_tables(m, re, nc, false, prec == MXM_PREC_FP32_MFMA);
+  ElemTables t = build_elem_tables(m, re, nc, false, prec == MXM_PREC_FP32_MFMA, kRoomBatch);
   *out = (long long)instance_bytes(t, m.NP, nc, m.NFP, dim, prec, limiter != 0);
   return MXM_OK;
 }

@@ -64,18 +64,24 @@ Connectivity build_connectivity(const HostMesh &m, const RefElem &re);
 // Element tiles of the stage kernel and the device element order.  A tile
 // is a block of lattice cells (squares of 2 triangles, cubes of 6 tets),
 // at most `epb` elements, whose shape minimises the face-flux work per
-// element (faces with both sides in the tile are evaluated once).  Device
+// element (faces with both sides in the tile are evaluated once); what
+// whole blocks leave over of a large mesh is cut into as few tiles as the
+// other shapes allow.  Device
 // element slot T*epb + el holds element ref_of[T*epb + el] (-1: padding),
 // so every tile is contiguous in device memory; dev_of is the inverse.
 // When one cell has more elements than a tile (3D, P = 5), tiles are runs
 // of consecutive elements and block = {0, 0, 0}.
 struct Tiling {
   int epb = 0, ntiles = 0;
-  int block[3] = {1, 1, 1};  // cells per tile along x, y, z
+  int block[3] = {1, 1, 1};  // cells of a whole block along x, y, z
   std::vector<int32_t> dev_of, ref_of, count;
   int slots() const { return ntiles * epb; }
 };
-Tiling build_tiling(const HostMesh &m, int epb, int NFP);
+// room: the most tiles that blocks cut off at the mesh's edge may make.
+// Alone on the device, one tile per CU; one of many, few, so that small
+// meshes of about the same size still take equal ranges of tiles.
+constexpr int kRoomAlone = 256, kRoomBatch = 16;
+Tiling build_tiling(const HostMesh &m, int epb, int NFP, int room);
 
 // Distinct face geometries of a lattice mesh, at most: 12 periodic face
 // types and 6 one-sided boundary ones in 3D, 3 and 2 in 2D.

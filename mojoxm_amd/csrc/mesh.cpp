@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <array>
 #include <cmath>
+#include <map>
 #include <stdexcept>
 
 #include "host.hpp"
@@ -475,14 +476,84 @@ Connectivity build_connectivity(const HostMesh &m, const RefElem &re) {
   return c;
 }
 
-Tiling build_tiling(const HostMesh &m, int epb, int NFP) {
+namespace {
+
+// Faces evaluated for a bx x by x bz block on a periodic lattice: pairs
+// inside the block once, faces to other blocks once per side.
+int block_faces(int dim, int bx, int by, int bz) {
+  const int inner = dim == 3 ? 6 : 1, per_iface = dim == 3 ? 2 : 1;
+  const int ifaces = (bx - 1) * by * bz + bx * (by - 1) * bz + (dim == 3 ? bx * by * (bz - 1) : 0);
+  const int sfaces = 2 * (by * bz + bx * bz + (dim == 3 ? bx * by : 0));
+  return bx * by * bz * inner + (ifaces + sfaces) * per_iface;
+}
+
+// Cuts the part of a lattice that whole blocks do not cover into tiles: a
+// region is filled with one block shape, and what that leaves over along x,
+// then y, then z is a smaller region of the same kind.  The shape (of at
+// most max_cells cells and max_faces faces) is the one that needs the
+// fewest tiles in all, then the one with the fewest faces per cell.
+struct RegionCutter {
+  struct Box {
+    int o[3], n[3];
+  };
+  struct Cut {
+    long long tiles = 0;
+    int b[3] = {0, 0, 0};
+  };
+  int dim, max_cells, max_faces;
+  std::map<std::array<int, 3>, Cut> memo;
+
+  // the regions that blocks b leave over in a region of X x Y x Z cells
+  static std::array<Box, 3> rest(const std::array<int, 3> &X, const int *b) {
+    const int w = X[0] - X[0] % b[0], h = X[1] - X[1] % b[1], d = X[2] - X[2] % b[2];
+    return {Box{{w, 0, 0}, {X[0] - w, X[1], X[2]}}, Box{{0, h, 0}, {w, X[1] - h, X[2]}},
+            Box{{0, 0, d}, {w, h, X[2] - d}}};
+  }
+  static long long whole(const std::array<int, 3> &X, const int *b) {
+    return (long long)(X[0] / b[0]) * (X[1] / b[1]) * (X[2] / b[2]);
+  }
+  Cut best(const std::array<int, 3> &X) {
+    Cut c;
+    if (!X[0] || !X[1] || !X[2]) return c;
+    const auto it = memo.find(X);
+    if (it != memo.end()) return it->second;
+    int cf = 0, cc = 0;
+    for (int bz = 1; bz <= X[2] && bz <= max_cells; ++bz)
+      for (int by = 1; by <= X[1] && by * bz <= max_cells; ++by)
+        for (int bx = 1; bx <= X[0] && bx * by * bz <= max_cells; ++bx) {
+          const int b[3] = {bx, by, bz}, nf = block_faces(dim, bx, by, bz), nc = bx * by * bz;
+          if (nf > max_faces) continue;
+          long long t = whole(X, b);
+          for (const Box &r : rest(X, b)) t += best({r.n[0], r.n[1], r.n[2]}).tiles;
+          if (!c.tiles || t < c.tiles || (t == c.tiles && nf * cc < cf * nc)) {
+            c.tiles = t, cf = nf, cc = nc;
+            std::copy(b, b + 3, c.b);
+          }
+        }
+    return memo[X] = c;
+  }
+  // the tiles of a region at o, cut with blocks b first
+  void cut(const int *o, const std::array<int, 3> &X, const int *b, std::vector<Box> &out) {
+    for (int z = 0; z + b[2] <= X[2]; z += b[2])
+      for (int y = 0; y + b[1] <= X[1]; y += b[1])
+        for (int x = 0; x + b[0] <= X[0]; x += b[0])
+          out.push_back({{o[0] + x, o[1] + y, o[2] + z}, {b[0], b[1], b[2]}});
+    for (const Box &r : rest(X, b)) {
+      const std::array<int, 3> n = {r.n[0], r.n[1], r.n[2]};
+      if (!n[0] || !n[1] || !n[2]) continue;
+      const int ro[3] = {o[0] + r.o[0], o[1] + r.o[1], o[2] + r.o[2]};
+      cut(ro, n, best(n).b, out);
+    }
+  }
+};
+
+}  // namespace
+
+Tiling build_tiling(const HostMesh &m, int epb, int NFP, int room) {
   if (epb < 1 || epb > 126) throw std::runtime_error("tiling: tile size out of range");
   const int dim = m.dim, epc = dim == 3 ? 6 : 2;  // elements per lattice cell
   const int nx = m.n[0], ny = m.n[1], nz = dim == 3 ? m.n[2] : 1;
   if ((long long)nx * ny * nz * epc != m.K) throw std::runtime_error("tiling: element count is not a lattice");
-  // Faces evaluated for a bx x by x bz block on a periodic lattice: pairs
-  // inside the block once, faces to other blocks once per side.
-  const int inner = dim == 3 ? 6 : 1, per_iface = dim == 3 ? 2 : 1;
   Tiling t;
   t.epb = epb;
   double best = 1e30;
@@ -492,9 +563,7 @@ Tiling build_tiling(const HostMesh &m, int epb, int NFP) {
       for (int bx = 1; bx <= nx; ++bx) {
         const int cells = bx * by * bz;
         if (cells * epc > epb) continue;
-        const int ifaces = (bx - 1) * by * bz + bx * (by - 1) * bz + (dim == 3 ? bx * by * (bz - 1) : 0);
-        const int sfaces = 2 * (by * bz + bx * bz + (dim == 3 ? bx * by : 0));
-        const int faces = cells * inner + ifaces * per_iface + sfaces * per_iface;
+        const int faces = block_faces(dim, bx, by, bz);
         // wave-executions of the face phase plus about one for the per-node
         // phases of the block, per element
         const int waves = (faces * NFP + 63) / 64;
@@ -519,28 +588,49 @@ Tiling build_tiling(const HostMesh &m, int epb, int NFP) {
     }
     return t;
   }
-  const int bx = t.block[0], by = t.block[1], bz = t.block[2];
-  const int tx = (nx + bx - 1) / bx, ty = (ny + by - 1) / by, tz = (nz + bz - 1) / bz;
-  t.ntiles = tx * ty * tz;
+  // Whole blocks, then smaller regions where the mesh is no multiple of the
+  // block.  Blocks cut off at the mesh's edge instead are partly filled
+  // tiles, which cost about what full ones do: 19^3 Taylor-Green (2 cells a
+  // tile) took 3610 tiles and 28.9 us a stage, now 3430 and 27.5; a batch of
+  // 24 GLM-MHD meshes of 17 to 87 squares 4750 (4502 would hold them), now
+  // 4545, and 28.4 -> 27.4 us.  While there are no more tiles than CUs, all
+  // of them run at once, a tile more costs nothing and a smaller one ends
+  // sooner, so blocks are cut off (16^2 GLM-MHD: 24 tiles 4.60 us, 22 4.71).
+  // No tile has more faces than a whole block, so that the job slots of a
+  // tile do not grow.  Tiles in the order of the whole blocks, x fastest;
+  // cells inside a tile z, y, x order; then the cell's elements.
+  const int *const b = t.block, origin[3] = {0, 0, 0};
+  std::vector<RegionCutter::Box> boxes;
+  const int tx = (nx + b[0] - 1) / b[0], ty = (ny + b[1] - 1) / b[1], tz = (nz + b[2] - 1) / b[2];
+  if ((long long)tx * ty * tz <= room) {
+    for (int z = 0; z < nz; z += b[2])
+      for (int y = 0; y < ny; y += b[1])
+        for (int x = 0; x < nx; x += b[0])
+          boxes.push_back({{x, y, z}, {std::min(b[0], nx - x), std::min(b[1], ny - y), std::min(b[2], nz - z)}});
+  } else {
+    RegionCutter{dim, epb / epc, best_faces, {}}.cut(origin, {nx, ny, nz}, b, boxes);
+  }
+  std::sort(boxes.begin(), boxes.end(), [&](const RegionCutter::Box &p, const RegionCutter::Box &q) {
+    const std::array<int, 5> kp = {p.o[2] / b[2], p.o[1] / b[1], p.o[0], p.o[1], p.o[2]};
+    return kp < std::array<int, 5>{q.o[2] / b[2], q.o[1] / b[1], q.o[0], q.o[1], q.o[2]};
+  });
+  t.ntiles = (int)boxes.size();
   t.ref_of.assign((size_t)t.ntiles * epb, -1);
   t.count.assign(t.ntiles, 0);
-  // tiles x-fastest; cells inside a tile z, y, x order; then the cell's elements
-  for (int TZ = 0; TZ < tz; ++TZ)
-    for (int TY = 0; TY < ty; ++TY)
-      for (int TX = 0; TX < tx; ++TX) {
-        const int T = (TZ * ty + TY) * tx + TX;
-        int el = 0;
-        for (int k = TZ * bz; k < std::min(nz, (TZ + 1) * bz); ++k)
-          for (int j = TY * by; j < std::min(ny, (TY + 1) * by); ++j)
-            for (int i = TX * bx; i < std::min(nx, (TX + 1) * bx); ++i)
-              for (int q = 0; q < epc; ++q) {
-                const int e = ((k * ny + j) * nx + i) * epc + q;
-                t.ref_of[(size_t)T * epb + el] = e;
-                t.dev_of[e] = T * epb + el;
-                ++el;
-              }
-        t.count[T] = el;
-      }
+  for (int T = 0; T < t.ntiles; ++T) {
+    const RegionCutter::Box &x = boxes[T];
+    int el = 0;
+    for (int k = x.o[2]; k < x.o[2] + x.n[2]; ++k)
+      for (int j = x.o[1]; j < x.o[1] + x.n[1]; ++j)
+        for (int i = x.o[0]; i < x.o[0] + x.n[0]; ++i)
+          for (int q = 0; q < epc; ++q) {
+            const int e = ((k * ny + j) * nx + i) * epc + q;
+            t.ref_of[(size_t)T * epb + el] = e;
+            t.dev_of[e] = T * epb + el;
+            ++el;
+          }
+    t.count[T] = el;
+  }
   for (int e = 0; e < m.K; ++e)
     if (t.dev_of[e] < 0) throw std::runtime_error("tiling: element not placed");
   return t;

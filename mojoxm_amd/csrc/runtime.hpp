@@ -230,11 +230,11 @@ struct ElemTables {
   std::vector<int> tile_type;  // cell element of each tile's first slot
 };
 
-// wide: tiles of the wide tile size (stage_epb)
-inline ElemTables build_elem_tables(const HostMesh &m, const RefElem &re, int nc, bool wide, bool fp32) {
+// wide: tiles of the wide tile size (stage_epb); room: see build_tiling
+inline ElemTables build_elem_tables(const HostMesh &m, const RefElem &re, int nc, bool wide, bool fp32, int room) {
   ElemTables t;
   Connectivity cn = build_connectivity(m, re);
-  t.til = build_tiling(m, stage_epb(m.dim, m.NP, m.NFP, nc, wide), m.NFP);
+  t.til = build_tiling(m, stage_epb(m.dim, m.NP, m.NFP, nc, wide), m.NFP, room);
   const int Kd = t.til.slots(), dd = m.dim * m.dim, NF = m.NF;
   t.invJ.assign((size_t)Kd * dd, 0.0);
   t.inv_vol.assign((size_t)Kd, 0.0);

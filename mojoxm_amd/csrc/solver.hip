@@ -169,7 +169,7 @@ struct Solver {
   // with a zero state and nothing pending; graphs are dropped
   void layout(const HostMesh &m, const RefElem &re) {
     drop_graphs();
-    ElemTables t = build_elem_tables(m, re, NC, wide, prec == MXM_PREC_FP32_MFMA);
+    ElemTables t = build_elem_tables(m, re, NC, wide, prec == MXM_PREC_FP32_MFMA, kRoomAlone);
     til = std::move(t.til);
     Kd = til.slots();
     ntiles = til.ntiles;
@@ -638,7 +638,8 @@ int mxm_mesh_create_3d(const mxm_mesh3d_desc *d, int P, void **mesh) {
     auto m = std::make_unique<HostMesh>(build_mesh_3d(d->nx, d->ny, d->nz, d->lx, d->ly, d->lz, d->bc, P, re));
     // the kernel-side tables are validated here too, so host-only callers
     // exercise the same checks a solver runs
-    build_face_jobs(*m, re, build_connectivity(*m, re), build_tiling(*m, stage_epb(m->dim, m->NP, m->NFP, 1), m->NFP));
+    build_face_jobs(*m, re, build_connectivity(*m, re), build_tiling(*m, stage_epb(m->dim, m->NP, m->NFP, 1), m->NFP,
+                                                                     kRoomAlone));
     *mesh = m.release();
     return MXM_OK;
   });
@@ -652,7 +653,8 @@ int mxm_mesh_create_2d(const mxm_mesh2d_desc *d, int P, void **mesh) {
     check_bc(d->bc, 4);
     RefElem re = build_refelem(2, P);
     auto m = std::make_unique<HostMesh>(build_mesh_2d(d->nx, d->ny, d->lx, d->ly, d->bc, P, re));
-    build_face_jobs(*m, re, build_connectivity(*m, re), build_tiling(*m, stage_epb(m->dim, m->NP, m->NFP, 1), m->NFP));
+    build_face_jobs(*m, re, build_connectivity(*m, re), build_tiling(*m, stage_epb(m->dim, m->NP, m->NFP, 1), m->NFP,
+                                                                     kRoomAlone));
     *mesh = m.release();
     return MXM_OK;
   });
