@@ -12,7 +12,7 @@
 // as one of its stored values is not finite (inst_fail, set by the stage
 // kernel), so instances with different step counts share the launches and
 // finished or failed ones cost a block exit.  One SSPRK3 step of a group
-// (three stages, limiter, counter bump) is a HIP graph, replayed.
+// (three stages, counter bump) is a HIP graph, replayed.
 //
 // Every group has its own HIP stream: groups (different physics, orders,
 // limiter settings) run concurrently on the device.  A new instance is

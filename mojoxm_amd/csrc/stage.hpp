@@ -12,10 +12,10 @@
 // One block (4 wave64, or 5 for the wide 2D P = 3 tile of the FP32-MFMA
 // form, below) per tile of at most EPB elements, which are contiguous in
 // device memory:
-//   1. each thread starts the loads of its first face item (job record
-//      with the face geometry, partner node, and the partner's trace when
-//      the partner lies outside the tile); the block stages the q_in tile
-//      and the tile's geometry in LDS;
+//   1. each thread starts the loads of its first face item (job record,
+//      partner node, and the partner's trace when the partner lies outside
+//      the tile); the block stages the q_in tile and the mesh's distinct
+//      face and cell geometries in LDS;
 //   2. per face item: the numerical flux (boundary faces: against the
 //      physics' ghost state), signed and scaled by the face area, into LDS.
 //      A face whose two elements are both in the tile is evaluated once by
@@ -24,8 +24,9 @@
 //      each side, as the reference evaluates every face from both sides;
 //      side 0 is always the left state.  Per (element, node): the nodal
 //      flux mapped to reference directions by invJ, into LDS;
-//   3. the D and Lift contractions over LDS, then per (element, node) the
-//      RK combine, limit_state and the store.
+//   3. the D and Lift contractions over LDS, the operator entries from the
+//      scalar cache (FP64) or straight to the MFMA's lanes (FP32), then per
+//      (element, node) the RK combine, limit_state and the store.
 //
 // Two arithmetic forms share the kernel:
 //   R = double  plain FP64: the contractions run on the VALU in FP64;
@@ -114,12 +115,11 @@ typedef const double __attribute__((address_space(4))) *ScalarPtr;
 // Launch configurations of the stage kernel: each is an occupancy target
 // (waves per SIMD, e.g. 256-thread blocks per CU) that bounds the register
 // allocation; all configurations compute the same bits.  The autotuner
-// times them on the problem and keeps the fastest.  FP64 kernels need
-// 100-150 VGPRs: 5 waves (<= 102 VGPRs) or 4 (<= 128, which takes the
-// 131-VGPR GLM-MHD kernel from 3 waves to 4); the FP32 kernels fit 5, 6
-// or 7 waves (<= 72 VGPRs: the 2D trait Euler kernel without spills), and
-// the compiler's own choice (1: no bound) can be far off (e.g. 250 VGPRs,
-// 1 wave, for the 2D Euler kernels at P = 1).
+// times them on the problem and keeps the fastest.  The FP64 kernels fit 5
+// waves (<= 102 VGPRs; the 2D HLLEC Euler kernel's 80 let 6 run) or 4
+// (<= 128: GLM-MHD); the FP32 kernels fit 5, 6 or 7 (<= 72 VGPRs), and the
+// compiler's own choice (1: no bound) can be far off (e.g. 250 VGPRs, 1
+// wave, for the 2D Euler kernels at P = 1).
 template <class R>
 struct StageCfg;
 template <>
@@ -139,7 +139,8 @@ constexpr int kStageCfgMax = 4;
 // tets) when a cell fits, then reduced -- by cells, then to runs of
 // elements -- until the block's LDS at FP64 (the operand array -- the q_in
 // tile and the face fluxes, later the ND*NP flux planes, rows of
-// EPB*NC + 1 values -- and the geometry) fits 64 KB, which only the
+// EPB*NC + 1 values -- and 8 bytes for each invJ entry and volume of the
+// elements, an allowance for the geometry) fits 64 KB, which only the
 // two-fluid state (NC = 17) needs.  Tiles are blocks of cells, so the LDS
 // is sized for what a tile can hold; the host builds the tiles with the
 // same value.
@@ -151,7 +152,7 @@ constexpr int kStageCfgMax = 4;
 // 24 triangles on 240 of 256 lanes, or 32 on all 320 lanes of 5 waves).
 // It pays when all tiles are resident at once: a mesh of 128 x 128
 // squares makes 1,024 wide tiles, 4 per CU and 5 waves per SIMD, against
-// 1,376 narrow ones, 5 or 6 per CU and 6 waves on the busiest SIMDs.
+// 1,370 narrow ones, 5 or 6 per CU and 6 waves on the busiest SIMDs.
 // When tiles queue for the CUs the narrow tile is faster (an 8-wave tile
 // of 50 triangles measured slower still): a CU then holds fewer, larger
 // blocks, whose barriers idle more waves at once and whose phases overlap
