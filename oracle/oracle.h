@@ -1,6 +1,6 @@
 /*
  * oracle.h -- CPU FP64 restatement of mojoxm's DG right-hand side and
- * SSPRK3 step.  TEST INFRASTRUCTURE ONLY: the checker that the HIP
+ * SSPRK3 step.  TEST INFRASTRUCTURE ONLY: what the HIP
  * library is compared against.  Nothing in the shipped library links,
  * loads or calls this code; only tests/, the smoke check and the CPU
  * baseline leg of bench.py do.
