@@ -54,22 +54,28 @@ __global__ __launch_bounds__(256) void bj_theta_kernel(double *__restrict__ thet
   theta[e0 + i] = bj_theta<NC, ALL, NF>(e0 + i, nb, mean, ext, eps2);
 }
 
-// the limited state written in place, then extrema equal to the means: a
-// block holds whole elements, one thread per node
+// the limited state written in place, then extrema equal to the means and
+// theta = 1 (a stage takes q_a's theta as it is stored): a block holds whole
+// elements, one thread per node, so every node has read theta before the
+// element's first thread resets it
 template <class R, int NC, bool ALL>
-__global__ __launch_bounds__(256) void bj_apply_kernel(R *__restrict__ q, const double *__restrict__ theta,
+__global__ __launch_bounds__(256) void bj_apply_kernel(R *__restrict__ q, double *__restrict__ theta,
                                                        const double *__restrict__ mean, double *__restrict__ ext,
                                                        int e0, int n, int NP) {
   constexpr int NCL = ALL ? NC : 1;
   const int epb = 256 / NP;
   const int el = threadIdx.x / NP, node = threadIdx.x - el * NP;
   const int i = blockIdx.x * epb + el;
-  if (el >= epb || i >= n) return;
+  const bool mine = el < epb && i < n;
   const size_t e = (size_t)e0 + i;
-  const double th = theta[e];
-  if (node == 0)
+  const double th = mine ? theta[e] : 1.0;
+  __syncthreads();
+  if (!mine) return;
+  if (node == 0) {
+    theta[e] = 1.0;
 #pragma unroll
     for (int c = 0; c < NCL; ++c) ext[(e * NCL + c) * 2] = ext[(e * NCL + c) * 2 + 1] = mean[e * NC + c];
+  }
   if (!(th < 1.0)) return;
   R *qn = q + (e * NP + node) * NC;
 #pragma unroll

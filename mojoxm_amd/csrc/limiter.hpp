@@ -13,9 +13,10 @@ constexpr int kLimMaxNC = 17;  // the widest state (two-fluid)
 // [slots][NCL][2] (smallest, largest node value of the limited components:
 // all NC in 3D, component 0 in 2D) and the neighbours' means through conn
 // (the partner slot of each of an element's NF faces); FP64 whatever the
-// state precision.  theta [slots] is scratch.  Afterwards nothing is pending
-// on these slots: their extrema equal their means, which makes their factor
-// 1.  The range covers every element of a mesh it touches.
+// state precision.  Afterwards nothing is pending on these slots: their
+// extrema equal their means, which makes their factor 1, and theta [slots],
+// which a stage reads for its q_a, is 1.  The range covers every element of
+// a mesh it touches.
 template <class R>
 hipError_t launch_bj_limit(R *q, double *theta, const double *mean, double *ext, const int *conn, int e0, int n,
                            int NP, int NC, int NF, int dim, double eps, hipStream_t s);
