@@ -724,10 +724,18 @@ dg_stage_kernel(StageArgs<R> A) {
   // 29.3, 113^2 P = 4 Maxwell 11.3 -> 11.0, 128^2 vortex 8.8 -> 8.6).
   constexpr int KL = (KPAD - KVP) / 4, KD = KVP / 4;      // k-steps of the lift and volume products
   constexpr bool kAhead = kMFMA && MT * (KL > KD ? KL : KD) <= 32;
+  constexpr int WAVES = S::BLOCK / 64, NTW = (NT + WAVES - 1) / WAVES;  // column tiles per wave
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // A wave without a column tile loads no operator and multiplies nothing.
+  // One component (or three at P = 5) leaves one to three of the block's
+  // waves without one; when they took part, the loads and MFMAs they
+  // repeated held up the other blocks (us per stage, 18^3 P = 3 advection
+  // 17.6 -> 10.8, 10^3 P = 5 36.4 -> 14.6, shallow water 37.4 -> 16.3).
+  const bool cols = NT > (WAVES - 1) * NTW || wave * NTW < NT;
   const int l = tid & 63, lr = l & 15, lg = l >> 4;
   auto aop = [&](int k, int m) { return A.Aop[(k * MT + m) * 64 + l]; };
   [[maybe_unused]] float al[kAhead ? KL : 1][MT], ad[kAhead ? KD : 1][MT];
-  if constexpr (kAhead) {
+  if (kAhead && cols) {
 #pragma unroll
     for (int k = 0; k < KL; ++k)
 #pragma unroll
@@ -746,8 +754,6 @@ dg_stage_kernel(StageArgs<R> A) {
   // columns [D (KVP) | Lift (KPAD - KVP)]; V_MFMA_F32_16X16X4F32 operands,
   // lane l = 16 g + r: A[r][k0 + g], B[k0 + g][col0 + r]; result rows
   // 4 g + v (v < 4), column col0 + r.
-  constexpr int NTW = (NT + S::BLOCK / 64 - 1) / (S::BLOCK / 64);  // column tiles per wave
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   mxm_float4 macc[kMFMA ? MT : 1][kMFMA ? NTW : 1];
   // FP64 on the VALU: the (element, component) columns are the lanes;
   // each wave group produces IH consecutive output nodes, so the operator
@@ -859,11 +865,13 @@ dg_stage_kernel(StageArgs<R> A) {
     for (int m = 0; m < MT; ++m)
 #pragma unroll
       for (int w = 0; w < NTW; ++w) macc[m][w] = mxm_float4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (kAhead) {
+    if (cols) {
+      if constexpr (kAhead) {
 #pragma unroll
-      for (int k = 0; k < KL; ++k) kstep(sS, al[k], k);
-    } else {
-      product(sS, KD, KD + KL);
+        for (int k = 0; k < KL; ++k) kstep(sS, al[k], k);
+      } else {
+        product(sS, KD, KD + KL);
+      }
     }
   } else {
 #pragma unroll
@@ -892,7 +900,7 @@ dg_stage_kernel(StageArgs<R> A) {
   }
   if constexpr (kMFMA && KVP > KV)
     for (int t = KV * NCOLS + tid; t < KVP * NCOLS; t += S::BLOCK) sB[t] = R(0);
-  if constexpr (kAhead) {
+  if (kAhead && cols) {
 #pragma unroll
     for (int k = 0; k < KD; ++k)
 #pragma unroll
@@ -902,11 +910,13 @@ dg_stage_kernel(StageArgs<R> A) {
 
   // ---- 3c. volume product, result as [el][i][c] ---------------------------
   if constexpr (kMFMA) {
-    if constexpr (kAhead) {
+    if (cols) {
+      if constexpr (kAhead) {
 #pragma unroll
-      for (int k = 0; k < KD; ++k) kstep(sW, ad[k], k);
-    } else {
-      product(sW, 0, KD);
+        for (int k = 0; k < KD; ++k) kstep(sW, ad[k], k);
+      } else {
+        product(sW, 0, KD);
+      }
     }
     __syncthreads();
 #pragma unroll
