@@ -383,8 +383,10 @@ dg_stage_kernel(StageArgs<R> A) {
   // 13.6 -> 13.1, 512^2 144 -> 138; 384^2 GLM-MHD FP64 110 -> 104, FP32 61.1
   // -> 59.6; limited 192^2 Sod FP64 32.5 -> 29.8).  The FP32 kernels of at
   // most 5 components fit 8 waves either way and keep the early load (512^2
-  // vortex 81.5, late 83.3).
-  constexpr bool kQaLate = !kMFMA || NC >= 6 || LIM;
+  // vortex 81.5, late 83.3), and so do the FP64 ones of P = 5 tets, whose
+  // blocks per CU the LDS bounds (small meshes, where nothing covers a wait:
+  // 4 x 5 x 4 Euler 26.7, early 25.5).
+  constexpr bool kQaLate = (kMFMA ? NC >= 6 : NP < 56) || LIM;
   constexpr int NB0 = stage_operand_len(kMFMA, TILE, NCOLS, KV, KVP, NFF, KPAD, NT * 16);
   // sW = sB: first the q_in tile as [el][j][c] (TILE contiguous values);
   // after the lift product the contravariant nodal fluxes as [k][j][el][c]
