@@ -772,13 +772,32 @@ dg_stage_kernel(StageArgs<R> A) {
 
   // acc[ii] += sum_r op[r][ii] col[r] over N rows: RB rows at a time, the next
   // rows' scalar and LDS loads in flight behind the FMAs of the present ones
-  // (two sets of RB*IH <= 16 operator entries in scalar registers).  Scalar
+  // (two sets of RB*IH operator entries in scalar registers).  Scalar
   // loads return out of order, so a wait for some is a wait for all: it
   // stands before the next rows are asked for.  Against one set, loaded and
   // waited for, us per stage: 512^2 vortex 149.7 -> 145.4, 128^2 14.1 -> 13.7,
   // 32^3 Taylor-Green 181 -> 176.5, 16^3 P = 2 advection 7.5 -> 6.7.
+  // A set holds up to 16 entries, and two rows of 9 or 10 where the product
+  // is longer than a 2D P = 3 one (20 rows): with one row of 10 a wave had 10
+  // FMAs to cover each wait (us per stage, one set / one row / two rows:
+  // 18^3 P = 3 Maxwell 51.4 / 58.3 / 49.1, MHD 71.5 / 81.5 / 66.9, 13^3 P = 4
+  // MHD 98 / 92 / 64; 100^2 P = 3 GLM-MHD 15.8 / 12.5 / 13.2).
+  // P = 5 tets, 14 entries a row from 75 KB of operator, have no room for two
+  // rows: with 3 to 9 components the plain loop, whose loads the compiler
+  // batches, is faster (10^3 Euler 76.0 / 76.1 / plain loop 73.5, MHD 84.6 /
+  // 97 / 79.3, Maxwell 72 / 72 / 65), with one or 17 this one (advection 124 /
+  // 81, two-fluid 480 / 304).
   [[maybe_unused]] auto contract = [&](const R *col, ScalarPtr op, auto N, double (&acc)[kMFMA ? 1 : IH]) {
-    constexpr int RB = IH <= 16 ? 16 / IH : 1, SETS = (N + RB - 1) / RB;
+    if constexpr (NP == 56 && NC > 1 && NC < 17) {
+#pragma unroll 4
+      for (int r = 0; r < N; ++r) {
+        const double v = col[r * NCOLS];
+#pragma unroll
+        for (int ii = 0; ii < IH; ++ii) acc[ii] += op[r * NPAD + ii] * v;
+      }
+      return;
+    }
+    constexpr int RB = IH <= 8 ? 16 / IH : IH <= 10 && N > 20 ? 2 : 1, SETS = (N + RB - 1) / RB;
     double o[2][RB][IH], v[2][RB];
     auto load = [&](int b, int s) {
 #pragma unroll
