@@ -31,36 +31,41 @@ __device__ __forceinline__ void bj_neighbours(int e, const int *conn, int (&nb)[
 #pragma unroll
   for (int f = 0; f < NF; ++f) nb[f] = conn[(size_t)e * NF + f];
 }
+// the smaller of th and the factor that component c asks for
+template <int NC, bool ALL, int NF>
+__device__ __forceinline__ double bj_theta_comp(int e, int c, const int (&nb)[NF], const double *mean,
+                                                const double *ext, double eps2, double th) {
+  constexpr int NCL = ALL ? NC : 1;
+  const double bm = mean[(size_t)e * NC + c];
+  double mn = bm, mx = bm;
+#pragma unroll
+  for (int f = 0; f < NF; ++f) {
+    const double v = mean[(size_t)nb[f] * NC + c];
+    if (ALL || nb[f] != e) {  // (its own mean constrains nothing)
+      mn = v < mn ? v : mn;
+      mx = v > mx ? v : mx;
+    }
+  }
+  const double pD = mx - bm < 0.0 ? 0.0 : mx - bm;
+  const double nD = bm - mn < 0.0 ? 0.0 : bm - mn;
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {  // the smallest and the largest node value
+    const double d = ext[((size_t)e * NCL + c) * 2 + s] - bm;
+    const double da = d >= 0.0 ? d : -d;
+    if (da <= 1.0e-30) continue;
+    const double D = d > 0.0 ? pD : nD;
+    const double D2 = D * D, d2 = da * da, Dd = D * da;
+    const double al = div_rounded(D2 + 2.0 * Dd + eps2, D2 + 2.0 * d2 + Dd + eps2);
+    th = al < th ? al : th;
+  }
+  return th;
+}
 template <int NC, bool ALL, int NF>
 __device__ __forceinline__ double bj_theta(int e, const int (&nb)[NF], const double *mean, const double *ext,
                                            double eps2) {
-  constexpr int NCL = ALL ? NC : 1;
   double th = 1.0;
 #pragma unroll
-  for (int c = 0; c < NCL; ++c) {
-    const double bm = mean[(size_t)e * NC + c];
-    double mn = bm, mx = bm;
-#pragma unroll
-    for (int f = 0; f < NF; ++f) {
-      const double v = mean[(size_t)nb[f] * NC + c];
-      if (ALL || nb[f] != e) {  // (its own mean constrains nothing)
-        mn = v < mn ? v : mn;
-        mx = v > mx ? v : mx;
-      }
-    }
-    const double pD = mx - bm < 0.0 ? 0.0 : mx - bm;
-    const double nD = bm - mn < 0.0 ? 0.0 : bm - mn;
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {  // the smallest and the largest node value
-      const double d = ext[((size_t)e * NCL + c) * 2 + s] - bm;
-      const double da = d >= 0.0 ? d : -d;
-      if (da <= 1.0e-30) continue;
-      const double D = d > 0.0 ? pD : nD;
-      const double D2 = D * D, d2 = da * da, Dd = D * da;
-      const double al = div_rounded(D2 + 2.0 * Dd + eps2, D2 + 2.0 * d2 + Dd + eps2);
-      th = al < th ? al : th;
-    }
-  }
+  for (int c = 0; c < (ALL ? NC : 1); ++c) th = bj_theta_comp<NC, ALL, NF>(e, c, nb, mean, ext, eps2, th);
   return th;
 }
 

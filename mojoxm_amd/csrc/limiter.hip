@@ -20,7 +20,10 @@
 // the factors that stage 1 stored.  As a launch of its own between two stages
 // theta took 3 to 5 us, latency for the most part, against 1 to 5 % more work
 // in the stage (us per limited stage, both before -> after: 75^2 P = 2 dam
-// break 10.9 -> 7.9, 48^2 Sod FP32 11.6 -> 7.6, 192^2 Sod FP64 33.3 -> 33.1).
+// break 10.9 -> 7.9, 48^2 Sod FP32 11.6 -> 7.6, 192^2 Sod FP64 33.3 -> 33.1;
+// in 3D, where all components are limited, 18^3 P = 3 Euler 66 -> 53, MHD 125
+// -> 109, two-fluid 432 -> 320, 28^3 P = 1 Euler 66 -> 58, two-fluid 391 -> 331;
+// dg_stage_kernel says how the block shares that work).
 // The kernels here limit a stored state in place for its other readers.
 //
 // The reference takes the minimum of the Venkatakrishnan factor

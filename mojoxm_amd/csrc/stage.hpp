@@ -413,8 +413,22 @@ dg_stage_kernel(StageArgs<R> A) {
   constexpr int NL = EPB * NC;
   __shared__ double sLim[LIM ? NL : 1];
   __shared__ double sTh[LIM ? EPB * (1 + NF) : 1];
+  // Where these slots alone do not fill the block and several components
+  // are limited, a thread takes one component of a slot at a time and the
+  // slot's factor is their minimum, formed in LDS (bit patterns of numbers
+  // that are not negative compare as integers); until the face fluxes, their
+  // rows hold each slot's element (-1: none) and neighbours.  A thread to a
+  // slot leaves the block waiting for the components one after another: us
+  // per limited stage, FP64, factors in a launch of their own / a thread to a
+  // slot / to a component: two-fluid 22^3 P = 2 345 / 442 / 307, 18^3 P = 3
+  // 432 / 501 / 319, 28^3 P = 1 391 / 495 / 331, MHD 18^3 P = 3 125 / 128 /
+  // 109, Euler 18^3 P = 3 66 / 58.4 / 53.5.  P = 1 with up to 6 components
+  // has more slots than threads (28^3 Euler 66 / 57.6 / 59.2).
+  constexpr bool kThetaComp = LIM && ND == 3 && NC > 1 && EPB * (1 + NF) <= S::BLOCK;
+  static_assert(!kThetaComp || EPB * (1 + NF) * (1 + NF) * sizeof(int) <= NFF * NCOLS * sizeof(R), "slots' neighbours");
   R *const sW = sB;
   R *const sS = sB + TILE;
+  [[maybe_unused]] int *const sNb = reinterpret_cast<int *>(sS);  // [slot][1 + NF] (kThetaComp)
 
   const int tid = threadIdx.x;
   const int tile = xcd_tile(blockIdx.x, A.ntiles);
@@ -458,8 +472,9 @@ dg_stage_kernel(StageArgs<R> A) {
   const int t2 = tid + S::BLOCK;
   [[maybe_unused]] FaceItem<R, NC> it2;
   if constexpr (kTwo) load_item_records<NFP, MAXT>(jobs, ipr, t2 < nitems ? t2 : nitems - 1, it2);
-  // limiter: thread i computes the factor of element i of the tile, then of
-  // the partner of face job i - EPB if that lies in another tile
+  // limiter: slot i of the factors, and thread i's part of their loads, is
+  // element i of the tile, then the partner of face job i - EPB if that lies
+  // in another tile
   const int thj = tid - EPB;
   int2 thjob = int2{-1, 0};
   if constexpr (LIM) thjob = jobs[thj < 0 ? 0 : thj < A.maxj ? thj : A.maxj - 1];
@@ -568,22 +583,43 @@ dg_stage_kernel(StageArgs<R> A) {
 #pragma unroll
     for (int k = 0; k < LPT; ++k)
       if (k * S::BLOCK + tid < NL) sLim[k * S::BLOCK + tid] = tl[k];
-    if (theta) {
-      const double th = bj_theta<NC, ND == 3, NF>(the, thnb, A.lim_mn_in, A.lim_ext_in, A.lim_eps2);
-      sTh[tid] = th;
-      if (thj < 0) A.lim_th_in[the] = th;
-    }
-    for (int i = tid + S::BLOCK; i < EPB + A.maxj; i += S::BLOCK) {  // more jobs than threads left
-      const int2 job = jobs[i - EPB];
-      if (job.x < 0 || (unsigned)(job.y - e0) < (unsigned)EPB) continue;
-      bj_neighbours<NF>(job.y, A.conn, thnb);
-      sTh[i] = bj_theta<NC, ND == 3, NF>(job.y, thnb, A.lim_mn_in, A.lim_ext_in, A.lim_eps2);
+    if constexpr (kThetaComp) {
+      if (tid < EPB * (1 + NF)) {
+        sTh[tid] = 1.0;
+        sNb[tid * (1 + NF)] = theta ? the : -1;
+#pragma unroll
+        for (int f = 0; f < NF; ++f) sNb[tid * (1 + NF) + 1 + f] = thnb[f];
+      }
+      __syncthreads();
+      for (int t = tid; t < (EPB + A.maxj) * NC; t += S::BLOCK) {
+        const int i = small_div<NC, EPB * (1 + NF) * NC>(t), e = sNb[i * (1 + NF)];
+        if (e < 0) continue;
+        int nb[NF];
+#pragma unroll
+        for (int f = 0; f < NF; ++f) nb[f] = sNb[i * (1 + NF) + 1 + f];
+        const double th = bj_theta_comp<NC, true, NF>(e, t - i * NC, nb, A.lim_mn_in, A.lim_ext_in, A.lim_eps2, 1.0);
+        if (th < 1.0)
+          atomicMin(reinterpret_cast<unsigned long long *>(&sTh[i]), (unsigned long long)__double_as_longlong(th));
+      }
+    } else {
+      if (theta) {
+        const double th = bj_theta<NC, ND == 3, NF>(the, thnb, A.lim_mn_in, A.lim_ext_in, A.lim_eps2);
+        sTh[tid] = th;
+        if (thj < 0) A.lim_th_in[the] = th;
+      }
+      for (int i = tid + S::BLOCK; i < EPB + A.maxj; i += S::BLOCK) {  // more jobs than threads left
+        const int2 job = jobs[i - EPB];
+        if (job.x < 0 || (unsigned)(job.y - e0) < (unsigned)EPB) continue;
+        bj_neighbours<NF>(job.y, A.conn, thnb);
+        sTh[i] = bj_theta<NC, ND == 3, NF>(job.y, thnb, A.lim_mn_in, A.lim_ext_in, A.lim_eps2);
+      }
     }
   }
   __syncthreads();
   // the q_in tile's pending limiter factors, applied in place to the
   // values this thread stored
   if constexpr (LIM) {
+    if (kThetaComp && tid < EPB) A.lim_th_in[e0 + tid] = sTh[tid];
 #pragma unroll
     for (int k = 0; k < QPT; ++k) {
       const int t = k * S::BLOCK + tid;
