@@ -1102,7 +1102,12 @@ hipError_t launch_stage(const void *args, hipStream_t s) {
     const StageArgs<R> &a = *static_cast<const StageArgs<R> *>(args);
     const int nb = a.ntiles;
     if (nb <= 0) return hipSuccess;
-    hipLaunchKernelGGL((dg_stage_kernel<Phys, ND, P, R, W, LIM, WIDE>), dim3(nb), dim3(S::BLOCK), 0, s, a);
+    // The 17 components of the two-fluid system spill 44 to 64 VGPRs of the
+    // FP32 kernels at 5 waves, where the LDS lets 5 be asked for; their
+    // 5-wave configuration is built for 4 (us per stage, 5 / 4 waves: 28^3
+    // P = 1 86 / 58, 22^3 P = 2 87 / 64, 18^3 P = 3 98 / 81, 10^3 P = 5 111 / 85).
+    constexpr int kWaves = std::is_same<R, float>::value && Phys::NC >= 17 && W == 5 ? 4 : W;
+    hipLaunchKernelGGL((dg_stage_kernel<Phys, ND, P, R, kWaves, LIM, WIDE>), dim3(nb), dim3(S::BLOCK), 0, s, a);
     return hipGetLastError();
   }
 }
