@@ -15,33 +15,55 @@
 #include <algorithm>
 #include <atomic>
 #include <cstdint>
+#include <cstdlib>
 #include <thread>
 #include <vector>
 
 namespace mxm {
 
-// Pinned buffers of the transfers of one solver or batch, kept between them.
+// Pinned buffers of the transfers of one solver or batch, kept between them
+// (pageable ones where no pinned memory can be had: the copies then wait).
 struct HostPieces {
   static constexpr size_t kPiece = 1 << 20;  // bytes of device state per piece
   static constexpr int kThreads = 8;         // at most; each has two pieces
   char *p = nullptr;
   int slots = 0;
+  bool pinned = false;
   hipEvent_t ev[2 * kThreads] = {};
+  HostPieces() = default;
+  HostPieces(const HostPieces &) = delete;
+  HostPieces &operator=(const HostPieces &) = delete;
   ~HostPieces() {
     for (auto e : ev)
       if (e) (void)hipEventDestroy(e);
-    if (p) (void)hipHostFree(p);
+    release();
+  }
+  void release() {
+    if (p && pinned)
+      (void)hipHostFree(p);
+    else
+      std::free(p);
+    p = nullptr, slots = 0;
   }
   hipError_t reserve(int n) {
+    for (int k = 0; k < n; ++k) {
+      if (ev[k]) continue;
+      const hipError_t e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
+      if (e != hipSuccess) {
+        ev[k] = nullptr;
+        return e;
+      }
+    }
     if (n <= slots) return hipSuccess;
-    char *q = nullptr;
-    hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&q), (size_t)n * kPiece);
-    if (e != hipSuccess) return e;
-    if (p) (void)hipHostFree(p);
-    p = q, slots = n;
-    for (int k = 0; k < n && e == hipSuccess; ++k)
-      if (!ev[k]) e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
-    return e;
+    release();
+    pinned = hipHostMalloc(reinterpret_cast<void **>(&p), (size_t)n * kPiece) == hipSuccess;
+    if (!pinned) {
+      (void)hipGetLastError();  // handled here, not the next launch's error
+      p = static_cast<char *>(std::malloc((size_t)n * kPiece));
+      if (!p) return hipErrorOutOfMemory;
+    }
+    slots = n;
+    return hipSuccess;
   }
 };
 
