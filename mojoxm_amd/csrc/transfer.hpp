@@ -67,6 +67,20 @@ struct HostPieces {
   }
 };
 
+// The device of a stream made current while its events are created: an event
+// belongs to the device that was current, and is recorded only on that
+// device's streams.
+struct OnDevice {
+  int before = -1, now;
+  explicit OnDevice(int device) : now(device) {
+    if (hipGetDevice(&before) != hipSuccess || before == now || hipSetDevice(now) != hipSuccess) before = now;
+  }
+  OnDevice(const OnDevice &) = delete;
+  ~OnDevice() {
+    if (before != now) (void)hipSetDevice(before);
+  }
+};
+
 // Slots [0, slots) of `dev` (node values each) <-> elements ref_of[slot] of h
 // (ref_of < 0: padding, zero on the device).  Returns when the caller may
 // use h (TO_HOST) or drop it, with the stream idle.
@@ -80,6 +94,7 @@ hipError_t move_state(HostPieces &hp, R *dev, const int32_t *ref_of, int slots, 
   // a thread pays from about two pieces on
   const int threads = std::max(1, std::min({HostPieces::kThreads, pieces / 2, (int)std::thread::hardware_concurrency()}));
   const int ring = pieces > threads ? 2 : 1;  // pieces each thread has under way
+  const OnDevice on(device);
   hipError_t e = hp.reserve(threads * ring);
   if (e != hipSuccess) return e;
   std::atomic<int> next{0}, error{(int)hipSuccess};
