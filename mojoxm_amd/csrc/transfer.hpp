@@ -27,7 +27,7 @@ struct HostPieces {
   static constexpr size_t kPiece = 1 << 20;  // bytes of device state per piece
   static constexpr int kThreads = 8;         // at most; each has two pieces
   char *p = nullptr;
-  int slots = 0;
+  size_t size = 0;
   bool pinned = false;
   hipEvent_t ev[2 * kThreads] = {};
   HostPieces() = default;
@@ -43,9 +43,10 @@ struct HostPieces {
       (void)hipHostFree(p);
     else
       std::free(p);
-    p = nullptr, slots = 0;
+    p = nullptr, size = 0;
   }
-  hipError_t reserve(int n) {
+  // n buffers, of `bytes` in all
+  hipError_t reserve(int n, size_t bytes) {
     for (int k = 0; k < n; ++k) {
       if (ev[k]) continue;
       const hipError_t e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
@@ -54,15 +55,16 @@ struct HostPieces {
         return e;
       }
     }
-    if (n <= slots) return hipSuccess;
+    if (bytes <= size) return hipSuccess;
+    bytes = std::max(bytes, std::min(2 * size, 2 * kThreads * kPiece));
     release();
-    pinned = hipHostMalloc(reinterpret_cast<void **>(&p), (size_t)n * kPiece) == hipSuccess;
+    pinned = hipHostMalloc(reinterpret_cast<void **>(&p), bytes) == hipSuccess;
     if (!pinned) {
       (void)hipGetLastError();  // handled here, not the next launch's error
-      p = static_cast<char *>(std::malloc((size_t)n * kPiece));
+      p = static_cast<char *>(std::malloc(bytes));
       if (!p) return hipErrorOutOfMemory;
     }
-    slots = n;
+    size = bytes;
     return hipSuccess;
   }
 };
@@ -95,7 +97,10 @@ hipError_t move_state(HostPieces &hp, R *dev, const int32_t *ref_of, int slots, 
   const int threads = std::max(1, std::min({HostPieces::kThreads, pieces / 2, (int)std::thread::hardware_concurrency()}));
   const int ring = pieces > threads ? 2 : 1;  // pieces each thread has under way
   const OnDevice on(device);
-  hipError_t e = hp.reserve(threads * ring);
+  // a small state takes what it needs: pinning a whole piece for it cost its
+  // first transfer 40 to 50 us (5^3 Euler, P = 2)
+  const size_t stride = ((size_t)std::min(per, slots) * node * sizeof(R) + 255) / 256 * 256;
+  hipError_t e = hp.reserve(threads * ring, (size_t)threads * ring * stride);
   if (e != hipSuccess) return e;
   std::atomic<int> next{0}, error{(int)hipSuccess};
   auto work = [&](int t) {
@@ -106,7 +111,7 @@ hipError_t move_state(HostPieces &hp, R *dev, const int32_t *ref_of, int slots, 
     if (t > 0 && !ok(hipSetDevice(device))) return;
     auto begin = [&](int c) { return c * per; };
     auto count = [&](int c) { return std::min(per, slots - c * per); };
-    auto buf = [&](int s) { return reinterpret_cast<R *>(hp.p + (size_t)(t * ring + s) * HostPieces::kPiece); };
+    auto buf = [&](int s) { return reinterpret_cast<R *>(hp.p + (size_t)(t * ring + s) * stride); };
     int piece[2] = {-1, -1};
     auto elements = [&](int c, R *b) {
       for (int k = 0; k < count(c); ++k) {

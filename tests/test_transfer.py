@@ -232,7 +232,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["sizes", "events", "pinned", "device", "copy"])
+@pytest.mark.parametrize("what", ["sizes", "events", "pinned", "device", "small", "copy"])
 def test_transfer(program, what):
     r = subprocess.run([program, what], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
