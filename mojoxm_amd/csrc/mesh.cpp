@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <array>
 #include <cmath>
+#include <cstring>
 #include <map>
 #include <stdexcept>
 
@@ -648,8 +649,10 @@ FaceJobs build_face_jobs(const HostMesh &m, const RefElem &re, const Connectivit
   auto geometry = [&](int fid) {
     double v[4] = {0.0, 0.0, 0.0, m.face_area[fid]};
     for (int d = 0; d < ND; ++d) v[d] = m.face_normal[(size_t)fid * ND + d];
+    // by their bits: what a mesh of extreme extents makes of them (an
+    // overflow, a NaN) is one geometry too
     for (int g = 0; g < ngeo; ++g)
-      if (std::equal(v, v + 4, &J.geo[(size_t)g * 4])) return g;
+      if (!std::memcmp(v, &J.geo[(size_t)g * 4], sizeof(v))) return g;
     if (ngeo == max_geo) throw std::runtime_error("jobs: more face geometries than a lattice has");
     std::copy(v, v + 4, &J.geo[(size_t)ngeo * 4]);
     return ngeo++;

@@ -71,3 +71,14 @@ def test_large_ragged_mesh_matches_the_oracle(oracle, P, n):
     got, want, _ = run_pair(oracle, n, (1.0, 0.8, 1.2)[:len(n)], P, EULER, None, nsteps=1, seed=P)
     assert np.isfinite(got).all()
     assert rel_l2(got, want) < TOL
+
+
+@pytest.mark.parametrize("precision", [M.PREC_FP64, M.PREC_FP32_MFMA])
+@pytest.mark.parametrize("L", [(1e155, 1e155, 1e-10), (1e160, 1e-100, 1e-100), (1e-100, 1e-100, 1e-100),
+                               (1e-155, 1e-155), (1e160, 1e160), (1.0 / 3.0, 7.3e-3), (0.7, 1e6, 3.1e-5)])
+def test_extreme_extents_are_accepted(L, precision):
+    """The geometry of a mesh is found again by its bits: extents whose face
+    normals overflow to NaN make tables as any others do."""
+    n = (3, 2, 5)[:len(L)]
+    for bc in (None, (M.BoundaryConditions(1, 2, 3, 1, 1, 2) if len(L) == 3 else M.BoundaryConditions2D(1, 2, 3, 1))):
+        assert footprint(n, L, EULER, 2, precision, bcs=bc) > 0
