@@ -411,8 +411,8 @@ struct Solver {
   }
 
   // enqueues the largest-signal-speed reduction of the current state on
-  // the solver's stream: tile maxima into part[ntiles], the maximum into
-  // out[0] (both device memory)
+  // the solver's stream: tile maxima into part[ntiles] (device memory), the
+  // maximum into out[0] (device memory, or pinned host memory)
   void enqueue_max_speed(double *part, double *out) {
     auto fill = [&](auto &a) {
       a.prm = dprm.p, a.tile_inst = nullptr, a.tile_count = tile_count.p;
@@ -434,7 +434,7 @@ struct Solver {
   // the largest signal speed over the nodes of the current state
   double max_wave_speed() {
     if (dpart.n < (size_t)ntiles) dpart.alloc(ntiles);
-    results.reserve(1);
+    results.reserve(3 * NC + 2);  // once for the diagnostics too: pinning took 26 us of their first call
     enqueue_max_speed(dpart.p, results.p);
     MXM_HIP(hipStreamSynchronize(stream));
     return results.p[0];
