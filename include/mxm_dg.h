@@ -86,9 +86,10 @@ extern "C" {
 /* Arithmetic of the stage kernels. */
 #define MXM_PREC_FP64 0      /* plain FP64 state, geometry and operators     */
 #define MXM_PREC_FP32_MFMA 1 /* FP32 state and fluxes, volume + LIFT on FP32
-                                MFMA with FP32 accumulation; geometry,
-                                Jacobians, RK combine, positivity rescue and
-                                limiter means in FP64                        */
+                                MFMA with FP32 accumulation; geometry and
+                                Jacobians formed in FP64 and rounded once;
+                                RK combine, positivity rescue and limiter
+                                means in FP64                                */
 
 /* ---- mesh descriptors -------------------------------------------------- */
 /* bc order [-x, +x, -y, +y, -z, +z], src/boundary.mojo:40-56 */
@@ -197,20 +198,27 @@ int mxm_dg_rk_stage(void *solver, int stage, double dt);
 /* nsteps x step_ssprk3, src/solver.mojo:1071-1092.  The steps are launched
  * as replayed HIP graphs, one of 32 steps and one of exactly the remainder
  * nsteps mod 32, rebuilt when dt, the limiter or the launch configuration
- * changed since the last call.  With the limiter on, each stage's factors
- * are applied by the next stage as it reads its inputs, and the limited
- * state is written at the end of the call: the state a caller sees is the
- * one per-stage limiting gives, bit for bit. */
+ * changed since the graphs were built.  Short calls launch their kernels on
+ * the solver's stream instead, which costs less than a graph or than
+ * building one to use it once: calls of 1 or 2 steps, and a call of up to 8
+ * steps whose dt (or other setting) has no graphs, unless the call before it
+ * that launched on the stream had the same dt.  The kernels and their
+ * results are the same either way.  With the limiter on, each stage computes
+ * and applies the factors pending on its inputs as it reads them, and the
+ * limited state is written at the end of the call: the state a caller sees
+ * is the one per-stage limiting gives, bit for bit. */
 int mxm_dg_step_ssprk3(void *solver, double dt, int nsteps);
-/* Builds the graphs mxm_dg_step_ssprk3(solver, dt, nsteps) replays, without
- * running a step (no reference counterpart: lets a caller keep graph
+/* Builds the graphs of mxm_dg_step_ssprk3(solver, dt, nsteps) without
+ * running a step, so that the call replays them; there are none to build for
+ * nsteps of 1 or 2 (no reference counterpart: lets a caller keep graph
  * construction out of a timed region). */
 int mxm_dg_prepare_steps(void *solver, double dt, int nsteps);
 /* enable_cell_limiter, src/solver.mojo:735-751 (eps: Venkatakrishnan). */
 int mxm_dg_enable_limiter(void *solver, int on, double eps);
 int mxm_dg_sync(void *solver);
 /* bench_step_loop, src/solver.mojo:765-802: warmup steps, sync, measure
- * steps, sync; advances the state by (warmup+measure)*dt. */
+ * steps, sync; advances the state by (warmup+measure)*dt.  Both run as
+ * replayed HIP graphs, whatever their length. */
 int mxm_dg_bench_step_loop(void *solver, double dt, int warmup, int measure,
                            mxm_throughput *out);
 /* dof_count / state_bytes_per_step / memory_report,
@@ -220,9 +228,8 @@ int mxm_dg_state_bytes_per_step(void *solver, long long *out);
 int mxm_dg_memory_report(void *solver, mxm_memory_report *out);
 /* Average duration (microseconds) of the stage kernel over 3*nsteps
  * back-to-back launches (limiter off), from two HIP events on the solver's
- * own stream around nsteps SSPRK3 steps launched as mxm_dg_step_ssprk3
- * launches them (replayed HIP graphs), so the average includes the
- * launch-to-launch gaps.  Before them, untimed: about 30 ms of steps (a
+ * own stream around nsteps SSPRK3 steps launched as replayed HIP graphs
+ * (whatever nsteps is), so the average includes the launch-to-launch gaps.  Before them, untimed: about 30 ms of steps (a
  * device coming out of idle clocks up over that much work) and the same
  * nsteps steps once, so the state advances by those steps and 2*nsteps.
  * No reference counterpart: it is the measurement hook that the roofline

@@ -79,7 +79,7 @@ struct Solver {
   int Kd = 0;  // device element slots, padding included
   int ntiles = 0;
 
-  // HIP graphs of SSPRK3 steps (kernel nodes only), replayed by step(): one
+  // HIP graphs of SSPRK3 steps (kernel nodes only), launched by replay(): one
   // of kGraphSteps steps and one of exactly r steps for each remainder
   // r = n mod kGraphSteps asked for, so step(n) is at most n / kGraphSteps
   // + 1 graph launches.  A graph bakes in dt, the limiter setting and the
@@ -443,7 +443,7 @@ struct Solver {
   // whether the graphs are those of the present settings and this dt
   bool graphs_current(double dt) const { return dt == g_dt && limiter == g_lim && eps == g_eps && cfg == g_cfg; }
 
-  // builds (if needed) the graphs that step(dt, n) replays
+  // builds (if needed) the graphs that replay(dt, n) launches
   void prepare(double dt, int n) {
     if (n <= 0) return;
     if (!graphs_current(dt)) {
@@ -455,6 +455,15 @@ struct Solver {
     if (r && !grem[r].exec) capture_steps(dt, r, grem[r]);
   }
 
+  // n steps as graph launches, whatever n
+  void replay(double dt, int n) {
+    if (n <= 0) return;
+    prepare(dt, n);
+    for (; n >= kGraphSteps; n -= kGraphSteps) MXM_HIP(hipGraphLaunch(gfull.exec, stream));
+    if (n) MXM_HIP(hipGraphLaunch(grem[n].exec, stream));
+    if (limiter) materialize(0);
+  }
+
   void step(double dt, int n) {
     if (n <= 0) return;
     if (n <= kDirectSteps || (n <= kFirstSteps && !graphs_current(dt) && dt != last_dt)) {
@@ -464,10 +473,7 @@ struct Solver {
       if (limiter) materialize(0);
       return;
     }
-    prepare(dt, n);
-    for (; n >= kGraphSteps; n -= kGraphSteps) MXM_HIP(hipGraphLaunch(gfull.exec, stream));
-    if (n) MXM_HIP(hipGraphLaunch(grem[n].exec, stream));
-    if (limiter) materialize(0);
+    replay(dt, n);
   }
 
   long long dof() const { return (long long)K * NP * NC; }
@@ -766,7 +772,7 @@ int mxm_dg_prepare_steps(void *h, double dt, int nsteps) {
   return guarded([&] {
     Solver *s = as_solver(h);
     if (nsteps < 0) throw ArgError("negative step count");
-    s->prepare(dt, nsteps);
+    if (nsteps > Solver::kDirectSteps) s->prepare(dt, nsteps);  // shorter calls replay no graph
     return MXM_OK;
   });
 }
@@ -802,13 +808,15 @@ int mxm_dg_bench_step_loop(void *h, double dt, int warmup, int measure, mxm_thro
   return guarded([&] {
     Solver *s = as_solver(h);
     if (!out || warmup < 0 || measure <= 0) throw ArgError("bad bench arguments");
-    s->step(dt, warmup);
+    // as graphs also where step() would launch on the stream: a warm-up that
+    // did would leave the capture of the measured steps inside their time
+    s->replay(dt, warmup);
     MXM_HIP(hipStreamSynchronize(s->stream));
     hipEvent_t ev[2];
     for (auto &e : ev) MXM_HIP(hipEventCreate(&e));
     auto t0 = std::chrono::steady_clock::now();
     MXM_HIP(hipEventRecord(ev[0], s->stream));
-    s->step(dt, measure);
+    s->replay(dt, measure);
     MXM_HIP(hipEventRecord(ev[1], s->stream));
     MXM_HIP(hipStreamSynchronize(s->stream));
     auto t1 = std::chrono::steady_clock::now();
@@ -884,16 +892,16 @@ int mxm_dg_time_stage_kernel(void *h, double dt, int nsteps, double *avg_us) {
     } restore{s, s->limiter};
     s->limiter = false;
     // two events on the solver's stream around nsteps SSPRK3 steps, launched
-    // as the stepping loop launches them (replayed graphs): the average
+    // as replayed graphs, as step() launches longer calls: the average
     // includes the launch-to-launch gaps.  Before the timed region the
     // device is warmed up and the same graphs run once, untimed.
     s->prepare(dt, nsteps);
     s->warm_up(dt, Solver::kWarmUpMs);
-    s->step(dt, nsteps);
+    s->replay(dt, nsteps);
     hipEvent_t ev[2];
     for (auto &e : ev) MXM_HIP(hipEventCreate(&e));
     MXM_HIP(hipEventRecord(ev[0], s->stream));
-    s->step(dt, nsteps);
+    s->replay(dt, nsteps);
     MXM_HIP(hipEventRecord(ev[1], s->stream));
     MXM_HIP(hipEventSynchronize(ev[1]));
     float ms = 0.f;

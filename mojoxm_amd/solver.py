@@ -106,8 +106,9 @@ class Solver:
         L.check(L.lib().mxm_dg_step_ssprk3(self._h, dt, nsteps), "mxm_dg_step_ssprk3")
 
     def prepare_steps(self, dt: float, nsteps: int) -> None:
-        """Build the replayed graphs step_ssprk3(dt, nsteps) uses, without
-        stepping (keeps graph construction out of a timed region)."""
+        """Build the graphs of step_ssprk3(dt, nsteps) without stepping, so that
+        the call replays them (keeps graph construction out of a timed
+        region); calls of 1 or 2 steps use none."""
         L.check(L.lib().mxm_dg_prepare_steps(self._h, dt, nsteps), "mxm_dg_prepare_steps")
 
     def enable_cell_limiter(self, enabled: bool = True, venkat_eps: float = 0.1) -> None:
