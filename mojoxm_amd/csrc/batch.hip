@@ -99,14 +99,15 @@ struct Arena {
   // [3][slots*NCL][2] (the limited components: all NC in 3D, component 0 in
   // 2D) and factors [3][slots] of the stage buffers
   DevBuf<double> lmean, ltheta, lext;
-  DevBuf<double> invJ, inv_vol, geom, iprm, idt, ipost;  // geom: one table per instance slot
+  DevBuf<double> geom, iprm, idt, ipost;  // geom, geomf: one table per instance slot
+  DevBuf<float> geomf;
   DevBuf<int> conn;  // limiter: partner slot per face
   DevBuf<int2> jobs;
   DevBuf<unsigned short> ipr;
   DevBuf<int> tile_count, tile_type, tile_inst, iactive, isteps, insteps, ifail;
   void swap(Arena &o) noexcept {
     for (int k = 0; k < 3; ++k) qd[k].swap(o.qd[k]), qf[k].swap(o.qf[k]);
-    lmean.swap(o.lmean), ltheta.swap(o.ltheta), lext.swap(o.lext), invJ.swap(o.invJ), inv_vol.swap(o.inv_vol), geom.swap(o.geom), iprm.swap(o.iprm);
+    lmean.swap(o.lmean), ltheta.swap(o.ltheta), lext.swap(o.lext), geom.swap(o.geom), geomf.swap(o.geomf), iprm.swap(o.iprm);
     idt.swap(o.idt), ipost.swap(o.ipost), conn.swap(o.conn), jobs.swap(o.jobs), ipr.swap(o.ipr);
     tile_count.swap(o.tile_count), tile_type.swap(o.tile_type), tile_inst.swap(o.tile_inst), iactive.swap(o.iactive), isteps.swap(o.isteps);
     insteps.swap(o.insteps), ifail.swap(o.ifail);
@@ -114,7 +115,7 @@ struct Arena {
   size_t bytes() const {
     size_t b = 0;
     for (int k = 0; k < 3; ++k) b += qd[k].bytes() + qf[k].bytes();
-    return b + lmean.bytes() + ltheta.bytes() + lext.bytes() + invJ.bytes() + inv_vol.bytes() + geom.bytes() + iprm.bytes() + idt.bytes() +
+    return b + lmean.bytes() + ltheta.bytes() + lext.bytes() + geom.bytes() + geomf.bytes() + iprm.bytes() + idt.bytes() +
            ipost.bytes() + conn.bytes() + jobs.bytes() + ipr.bytes() + tile_count.bytes() + tile_type.bytes() + tile_inst.bytes() +
            iactive.bytes() + isteps.bytes() + insteps.bytes() + ifail.bytes();
   }
@@ -240,11 +241,11 @@ size_t instance_bytes(const ElemTables &t, int NP, int NC, int NFP, int dim, int
   const size_t slots = (size_t)t.til.slots(), tiles = (size_t)t.til.ntiles, js = tiles * t.fj.maxj;
   const size_t word = prec == MXM_PREC_FP64 ? sizeof(double) : sizeof(float);
   size_t b = 3 * slots * NP * NC * word;                            // state trio
-  b += slots * (dim * dim + 1) * sizeof(double);                    // invJ, inv_vol
   b += slots * (dim + 1) * sizeof(int);                             // limiter neighbours
   b += js * (sizeof(int2) + NFP * sizeof(unsigned short));          // jobs, partner nodes
   b += tiles * 3 * sizeof(int);                                     // tile_count, tile_type, tile_inst
-  b += (MXM_PRM_MAX + 2 + t.geom.size()) * sizeof(double) + 4 * sizeof(int);  // per-instance scalars, geometry
+  b += (MXM_PRM_MAX + 2) * sizeof(double) + 4 * sizeof(int);        // per-instance scalars
+  b += t.geom.size() * sizeof(double) + t.geomf.size() * sizeof(float);
   if (limiter) b += slots * (3 * NC + 6 * (dim == 3 ? NC : 1) + 3) * sizeof(double);  // means, factors, extrema
   return b;
 }
@@ -252,7 +253,8 @@ size_t instance_bytes(const ElemTables &t, int NP, int NC, int NFP, int dim, int
 // Host images of one instance's tables at its place in an arena (base
 // tile bt, slot sl, maxj job slots per tile), in the arena's layouts.
 struct InstImage {
-  std::vector<double> ij, iv, geo, prm;
+  std::vector<double> geo, prm;
+  std::vector<float> geof;
   std::vector<int> cn;
   std::vector<int2> jb;
   std::vector<unsigned short> pr;
@@ -264,15 +266,14 @@ struct InstImage {
 InstImage inst_image(const BGroup &g, const BInst &in, int bt, int sl, int maxj) {
   InstImage m;
   const ElemTables &t = in.t;
-  const int epb = g.epb, dd = g.dim * g.dim, NF = g.NF, NFP = g.NFP;
+  const int epb = g.epb, NF = g.NF, NFP = g.NFP;
   const int lt = t.til.ntiles, lmj = t.fj.maxj, bs = bt * epb;
   const size_t slots = (size_t)lt * epb;
-  m.ij.assign(t.invJ.begin(), t.invJ.begin() + slots * dd);
-  m.iv.assign(t.inv_vol.begin(), t.inv_vol.begin() + slots);
   m.cn.resize(slots * NF);
   for (size_t s = 0; s < slots * NF; ++s) m.cn[s] = t.conn[s] + bs;
   m.jb.resize((size_t)lt * maxj);
   m.geo = t.geom;
+  m.geof = t.geomf;
   m.ty = t.tile_type;
   m.pr.assign((size_t)lt * maxj * NFP, 0);
   m.tc.resize(lt);
@@ -505,7 +506,7 @@ struct Batch {
   void upload_instance(BGroup &g, DevBuf<R> (&q)[3], BInst &in, int bt, int sl) {
     const InstImage m = inst_image(g, in, bt, sl, g.maxj);
     const std::vector<R> qs = device_state<R>(g, in);
-    const int dd = g.dim * g.dim, NF = g.NF;
+    const int NF = g.NF;
     const size_t bs = (size_t)bt * g.epb;
     struct Seg {
       void *dst;
@@ -514,11 +515,10 @@ struct Batch {
     };
     const Seg segs[] = {
         {q[0].p + bs * g.NP * g.NC, qs.data(), qs.size() * sizeof(R)},
-        {g.ar.invJ.p + bs * dd, m.ij.data(), m.ij.size() * sizeof(double)},
-        {g.ar.inv_vol.p + bs, m.iv.data(), m.iv.size() * sizeof(double)},
         {g.ar.conn.p + bs * NF, m.cn.data(), m.cn.size() * sizeof(int)},
         {g.ar.jobs.p + (size_t)bt * g.maxj, m.jb.data(), m.jb.size() * sizeof(int2)},
         {g.ar.geom.p + (size_t)sl * m.geo.size(), m.geo.data(), m.geo.size() * sizeof(double)},
+        {g.ar.geomf.p + (size_t)sl * m.geof.size(), m.geof.data(), m.geof.size() * sizeof(float)},
         {g.ar.ipr.p + (size_t)bt * g.maxj * g.NFP, m.pr.data(), m.pr.size() * sizeof(unsigned short)},
         {g.ar.tile_count.p + bt, m.tc.data(), m.tc.size() * sizeof(int)},
         {g.ar.tile_type.p + bt, m.ty.data(), m.ty.size() * sizeof(int)},
@@ -535,6 +535,7 @@ struct Batch {
     Staging &st = stage_buf(total);
     size_t off = 0;
     for (const Seg &s : segs) {
+      if (!s.bytes) continue;  // a table of the other form
       std::memcpy(st.p + off, s.src, s.bytes);
       MXM_HIP(hipMemcpyAsync(s.dst, st.p + off, s.bytes, hipMemcpyHostToDevice, g.stream));
       off += (s.bytes + 15) / 16 * 16;
@@ -625,7 +626,7 @@ struct Batch {
     const int ni = (int)order.size();
     const int cap_slots = ni + 1 + (grow ? std::max(8, (int)(ni * headroom)) : 0);
     const int cap_tiles = std::max(1, tiles + (grow ? (int)(tiles * headroom) : 0));
-    const int epb = g.epb, dd = g.dim * g.dim, NF = g.NF, NFP = g.NFP;
+    const int epb = g.epb, NF = g.NF, NFP = g.NFP;
     const size_t slots = (size_t)cap_tiles * epb, tile_vals = (size_t)epb * g.NP * g.NC;
     Arena na;
     auto state_trio = [&](auto &nq, auto &oq) {
@@ -653,9 +654,11 @@ struct Batch {
       state_trio(na.qd, g.ar.qd);
     else
       state_trio(na.qf, g.ar.qf);
-    std::vector<double> ij(slots * dd, 0.0), iv(slots, 0.0);
-    const size_t gl = stage_geom_len(g.dim, g.prec == MXM_PREC_FP32_MFMA);
+    const bool fp32 = g.prec == MXM_PREC_FP32_MFMA;
+    const size_t gl = fp32 ? cell_geom_len(g.dim) : stage_geom_len(g.dim, false);
+    const size_t glf = fp32 ? stage_geom_len(g.dim, true) : 0;
     std::vector<double> geo(cap_slots * gl, 0.0);
+    std::vector<float> geof(cap_slots * glf, 0.f);
     std::vector<int> cn(slots * NF);
     std::vector<int2> jb((size_t)cap_tiles * maxj);
     std::vector<unsigned short> pr((size_t)cap_tiles * maxj * NFP, 0);
@@ -673,11 +676,10 @@ struct Batch {
       const int sl = k + 1;
       const InstImage m = inst_image(g, in, bt, sl, maxj);
       const size_t bs = (size_t)bt * epb;
-      std::copy(m.ij.begin(), m.ij.end(), ij.begin() + bs * dd);
-      std::copy(m.iv.begin(), m.iv.end(), iv.begin() + bs);
       std::copy(m.cn.begin(), m.cn.end(), cn.begin() + bs * NF);
       std::copy(m.jb.begin(), m.jb.end(), jb.begin() + (size_t)bt * maxj);
       std::copy(m.geo.begin(), m.geo.end(), geo.begin() + (size_t)sl * gl);
+      std::copy(m.geof.begin(), m.geof.end(), geof.begin() + (size_t)sl * glf);
       std::copy(m.pr.begin(), m.pr.end(), pr.begin() + (size_t)bt * maxj * NFP);
       std::copy(m.tc.begin(), m.tc.end(), tc.begin() + bt);
       std::copy(m.ty.begin(), m.ty.end(), ty.begin() + bt);
@@ -687,11 +689,10 @@ struct Batch {
       new_base[k] = bt;
       bt += in.ntiles();
     }
-    na.invJ.upload(ij.data(), ij.size());
-    na.inv_vol.upload(iv.data(), iv.size());
     na.conn.upload(cn.data(), cn.size());
     na.jobs.upload(jb.data(), jb.size());
     na.geom.upload(geo.data(), geo.size());
+    na.geomf.upload(geof.data(), geof.size());
     na.ipr.upload(pr.data(), pr.size());
     na.tile_count.upload(tc.data(), tc.size());
     na.tile_type.upload(ty.data(), ty.size());
@@ -808,7 +809,10 @@ struct Batch {
     // GLM decay per instance (factor 1 where alpha_d = 0)
     a.post_comp = s == 2 && g.phys == MXM_PHYS_MHDGLM2D ? 6 : -1;
     a.tile_count = ar.tile_count.p, a.tile_type = ar.tile_type.p;
-    a.geom = ar.geom.p;
+    if constexpr (std::is_same<R, double>::value)
+      a.geom = ar.geom.p;
+    else
+      a.geom = ar.geomf.p;
     a.Dt = g.Dt.p, a.Lt = g.Lt.p, a.Aop = g.Aop.p, a.fmap = g.fmap.p;
     a.jobs = ar.jobs.p, a.ipr = ar.ipr.p, a.maxj = g.maxj, a.ntiles = g.grid_tiles;
     return a;
@@ -1018,7 +1022,9 @@ struct Batch {
     if (g.dpart.n < (size_t)nt * per) g.dpart.alloc((size_t)nt * per);
     if (g.dout.n < (size_t)(3 * NC + 2)) g.dout.alloc(3 * NC + 2);
     auto fill = [&](auto &a) {
-      a.invJ = g.ar.invJ.p, a.inv_vol = g.ar.inv_vol.p, a.w = g.w.p, a.Dn = g.Dn.p, a.tile_count = g.ar.tile_count.p;
+      const size_t gl = in.t.geom.size(), cell = cell_geom_len(g.dim);
+      a.cell = g.ar.geom.p + (in.slot + 1) * gl - cell, a.tile_type = g.ar.tile_type.p;
+      a.w = g.w.p, a.Dn = g.Dn.p, a.tile_count = g.ar.tile_count.p;
       a.epb = g.epb, a.tile0 = in.base_tile, a.ntiles = nt, a.NC = NC, a.nvel = diag_nvel(g.phys);
       a.part = g.dpart.p, a.pmax = g.dpart.p + (size_t)nt * kDiagSums * 2, a.out = g.dout.p;
     };

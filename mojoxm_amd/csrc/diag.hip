@@ -73,6 +73,7 @@ __global__ __launch_bounds__(B) void diag_tile_kernel(DiagArgs<R> A) {
   const bool node = tid < nE * NP;
   const int el = tid / NP, i = tid - el * NP;
   const size_t slot = (size_t)T * A.epb + el;
+  const double *const iJ = A.cell + (A.tile_type[T] + el) % cell_elems(ND) * cell_geom_elem(ND);
   double qv[kDiagMaxNC];
   double vw = 0.0;  // V_e w_i
 #pragma unroll
@@ -80,7 +81,7 @@ __global__ __launch_bounds__(B) void diag_tile_kernel(DiagArgs<R> A) {
   if (node) {
     const R *g = A.q + slot * NP * NC + (size_t)i * NC;
     for (int c = 0; c < NC; ++c) qv[c] = double(g[c]);
-    vw = kRefVol / A.inv_vol[slot] * A.w[i];
+    vw = kRefVol / iJ[ND * ND] * A.w[i];
   }
   if (A.nvel > 0 && node) {
     const double r = qv[0];
@@ -90,7 +91,6 @@ __global__ __launch_bounds__(B) void diag_tile_kernel(DiagArgs<R> A) {
   __syncthreads();
   double ke = 0.0, ens = 0.0;
   if (A.nvel > 0 && node) {
-    const double *iJ = A.invJ + slot * ND * ND;
     double g[3][3] = {{0.0}};  // g[a][b] = d u_a / d x_b
     for (int k = 0; k < ND; ++k) {
       const double *Dk = A.Dn + ((size_t)k * NP + i) * NP;

@@ -11,8 +11,8 @@ constexpr int kDiagSums = 2 * kDiagMaxNC + 2;   // per-tile sums: q_c, q_c^2, KE
 template <class R>
 struct DiagArgs {
   const R *q;             // [slots][NP][NC], tile-ordered state
-  const double *invJ;     // [slots][ND*ND], rows = reference directions
-  const double *inv_vol;  // [slots] 1/(6V) or 1/(2A)
+  const double *cell;     // geometry of the elements of a lattice cell (cell_geom_len)
+  const int *tile_type;   // [tiles] cell element of the tile's first slot
   const double *w;        // [NP] node weights, sum 1
   const double *Dn;       // [ND][NP][NP] nodal differentiation, d phi_j / d r_k at node i
   const int *tile_count;  // [tiles] elements per tile

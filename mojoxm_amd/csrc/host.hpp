@@ -88,6 +88,10 @@ Tiling build_tiling(const HostMesh &m, int epb, int NFP, int room);
 constexpr int max_face_geo(int dim) { return dim == 3 ? 18 : 5; }
 // Elements of a lattice cell
 constexpr int cell_elems(int dim) { return dim == 3 ? 6 : 2; }
+// Geometry of the elements of a lattice cell in FP64: invJ (rows = reference
+// directions), then inv_vol, of each
+constexpr int cell_geom_elem(int dim) { return dim * dim + 1; }
+constexpr int cell_geom_len(int dim) { return cell_elems(dim) * cell_geom_elem(dim); }
 // Length of the stage kernel's geometry table (StageArgs::geom), and of an
 // element's part of it
 constexpr int stage_geom_elem(int dim, bool fp32) { return dim * dim + (fp32 ? max_face_geo(dim) : 1); }

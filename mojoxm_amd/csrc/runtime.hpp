@@ -221,12 +221,13 @@ inline StagePlan stage_plan(int s) {
 struct ElemTables {
   Tiling til;
   FaceJobs fj;
-  std::vector<double> invJ, inv_vol;
   std::vector<int> conn;  // limiter neighbours: the partner slot of each face (its own slot on a boundary)
   // the stage kernel's geometry (StageArgs::geom): the distinct face normals
   // and areas, then invJ and inv_vol (FP32 form: -inv_vol times each area) of
-  // each element of a lattice cell
+  // each element of a lattice cell; the FP32 form's is rounded once, in geomf,
+  // and its geom holds the cell's elements alone (cell_geom_len)
   std::vector<double> geom;
+  std::vector<float> geomf;
   std::vector<int> tile_type;  // cell element of each tile's first slot
 };
 
@@ -236,8 +237,6 @@ inline ElemTables build_elem_tables(const HostMesh &m, const RefElem &re, int nc
   Connectivity cn = build_connectivity(m, re);
   t.til = build_tiling(m, stage_epb(m.dim, m.NP, m.NFP, nc, wide), m.NFP, room);
   const int Kd = t.til.slots(), dd = m.dim * m.dim, NF = m.NF;
-  t.invJ.assign((size_t)Kd * dd, 0.0);
-  t.inv_vol.assign((size_t)Kd, 0.0);
   t.conn.resize((size_t)Kd * NF);
   // a padding slot is its own neighbour with a zero state, which the
   // limiter leaves unchanged
@@ -247,17 +246,21 @@ inline ElemTables build_elem_tables(const HostMesh &m, const RefElem &re, int nc
       const int32_t *c = &cn.conn[((size_t)(e < 0 ? 0 : e) * NF + lf) * 4];
       t.conn[(size_t)sl * NF + lf] = e < 0 ? sl : t.til.dev_of[c[0]];
     }
-    if (e < 0) continue;
-    for (int k = 0; k < dd; ++k) t.invJ[(size_t)sl * dd + k] = m.elem_invJ[(size_t)e * dd + k];
-    t.inv_vol[sl] = m.elem_inv_vol[e];
   }
   t.fj = build_face_jobs(m, re, cn, t.til);
-  t.geom = std::move(t.fj.geo);
   const int epc = cell_elems(m.dim);
+  const std::vector<double> faces = std::move(t.fj.geo);
+  if (fp32)
+    t.geomf.assign(faces.begin(), faces.end());
+  else
+    t.geom = faces;
   for (int y = 0; y < epc; ++y) {
-    t.geom.insert(t.geom.end(), &m.elem_invJ[(size_t)y * dd], &m.elem_invJ[(size_t)y * dd] + dd);
-    if (!fp32) t.geom.push_back(m.elem_inv_vol[y]);
-    for (int g = 0; fp32 && g < max_face_geo(m.dim); ++g) t.geom.push_back(-m.elem_inv_vol[y] * t.geom[4 * g + 3]);
+    const double *iJ = &m.elem_invJ[(size_t)y * dd], iv = m.elem_inv_vol[y];
+    t.geom.insert(t.geom.end(), iJ, iJ + dd);
+    t.geom.push_back(iv);
+    if (!fp32) continue;
+    t.geomf.insert(t.geomf.end(), iJ, iJ + dd);
+    for (int g = 0; g < max_face_geo(m.dim); ++g) t.geomf.push_back(float(-iv * faces[4 * g + 3]));
   }
   // every element has the geometry of its place in its cell, and a tile's
   // slots run through those places in order

@@ -63,10 +63,10 @@ struct Solver {
   // components: all NC in 3D, component 0 in 2D) and factors [3][Kd] of the
   // stage buffers (q, q1, q2)
   DevBuf<double> lmean, ltheta, lext;
-  DevBuf<double> invJ, inv_vol, geom, Dt, Lt, w, dprm;
+  DevBuf<double> geom, Dt, Lt, w, dprm;
   DevBuf<double> Dn, dpart;  // diagnostics: nodal derivative, tile partials
   PinBuf results;            // diagnostics and speed, written by the kernels
-  DevBuf<float> Aop;
+  DevBuf<float> geomf, Aop;  // geomf: the FP32 stage kernel's (ElemTables)
   DevBuf<int> conn;  // limiter: partner slot per face
   DevBuf<int> fmap, tile_count, tile_type;
   DevBuf<int2> jobs;
@@ -189,14 +189,13 @@ struct Solver {
     lext.alloc((size_t)3 * 2 * Kd * ncl());
     ltheta.alloc((size_t)3 * Kd);
     if (limiter) clear_pending();
-    invJ.upload(t.invJ.data(), t.invJ.size());
-    inv_vol.upload(t.inv_vol.data(), t.inv_vol.size());
     conn.upload(t.conn.data(), t.conn.size());
     maxj = t.fj.maxj;
     tile_count.upload(til.count.data(), til.count.size());
     tile_type.upload(t.tile_type.data(), t.tile_type.size());
     jobs.upload(reinterpret_cast<const int2 *>(t.fj.jobs.data()), t.fj.jobs.size() / 2);
     geom.upload(t.geom.data(), t.geom.size());
+    if (!t.geomf.empty()) geomf.upload(t.geomf.data(), t.geomf.size());
     ipr.upload(t.fj.ipr.data(), t.fj.ipr.size());
     MXM_HIP(hipDeviceSynchronize());
   }
@@ -259,7 +258,10 @@ struct Solver {
     a.inst_prm = dprm.p;  // one instance: tile_inst, inst_dt, inst_post, inst_active stay null
     a.dt = dt;
     a.tile_count = tile_count.p, a.tile_type = tile_type.p;
-    a.geom = geom.p;
+    if constexpr (std::is_same<R, double>::value)
+      a.geom = geom.p;
+    else
+      a.geom = geomf.p;
     a.Dt = Dt.p, a.Lt = Lt.p, a.Aop = Aop.p, a.fmap = fmap.p;
     a.jobs = jobs.p, a.ipr = ipr.p, a.maxj = maxj, a.ntiles = ntiles;
     a.post_comp = s == 2 ? post_component(phys, prm) : -1;
@@ -390,7 +392,8 @@ struct Solver {
     if (dpart.n < (size_t)ntiles * per) dpart.alloc((size_t)ntiles * per);
     results.reserve(3 * NC + 2);
     auto fill = [&](auto &a) {
-      a.invJ = invJ.p, a.inv_vol = inv_vol.p, a.w = w.p, a.Dn = Dn.p, a.tile_count = tile_count.p;
+      a.cell = geom.p + geom.n - cell_geom_len(dim), a.tile_type = tile_type.p;
+      a.w = w.p, a.Dn = Dn.p, a.tile_count = tile_count.p;
       a.epb = til.epb, a.tile0 = 0, a.ntiles = ntiles, a.NC = NC, a.nvel = diag_nvel(phys);
       a.part = dpart.p, a.pmax = dpart.p + (size_t)ntiles * kDiagSums * 2, a.out = results.p;
     };
@@ -871,8 +874,7 @@ int mxm_dg_memory_report(void *h, mxm_memory_report *o) {
     o->rk_stage = (long long)s->state_bytes();
     o->dg_operators = (long long)(s->Dt.bytes() + s->Lt.bytes() + s->Aop.bytes() + s->w.bytes() + s->fmap.bytes());
     o->limiter = (long long)(s->lmean.bytes() + s->ltheta.bytes() + s->lext.bytes());
-    o->mesh_connectivity = (long long)(s->invJ.bytes() + s->inv_vol.bytes() + s->conn.bytes() +
-                                       s->geom.bytes() + s->tile_type.bytes() + s->jobs.bytes() + s->ipr.bytes() +
+    o->mesh_connectivity = (long long)(s->conn.bytes() + s->geom.bytes() + s->geomf.bytes() + s->tile_type.bytes() + s->jobs.bytes() + s->ipr.bytes() +
                                        s->tile_count.bytes());
     o->halo_device = 0;
     o->halo_pinned = 0;

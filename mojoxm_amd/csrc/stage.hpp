@@ -87,7 +87,7 @@ struct StageArgs {
   double dt, post_scale;
   int post_comp;            // component scaled after the combine (GLM psi: Phys::kPost), -1 none
   const int *tile_count;  // [ntiles] elements in each tile (slots T*EPB ..)
-  const double *geom;     // [n_inst][stage_geom_len]: the mesh's distinct face normals and areas
+  const R *geom;          // [n_inst][stage_geom_len]: the mesh's distinct face normals and areas
                           // ([max_face_geo][4]), then per element of a lattice cell invJ (ND*ND, rows =
                           // reference directions) and inv_vol (1/(6V) or 1/(2A)), in the FP32 form
                           // -inv_vol times each of those areas
@@ -395,12 +395,12 @@ dg_stage_kernel(StageArgs<R> A) {
   __shared__ __align__(16) R sB[NB0];
   // the geometry (StageArgs::geom): face normals and areas, then invJ and
   // inv_vol of each element of a lattice cell.  A lattice has a handful of
-  // each, so a tile reads 0.2 to 1 KB for them, the same for every tile,
+  // each, so a tile reads 0.15 to 1.1 KB for them, the same for every tile,
   // where a record per face and per slot took 3 KB: 77 of the 251 MB that
   // the FP32 512^2 vortex stage fetched (90.6 -> 86.0 us; 32^3 Taylor-Green
   // FP64 186 -> 181, 16^3 P = 2 advection 7.9 -> 7.5).
-  // The FP32 form keeps its table in FP32 with the face scales multiplied
-  // out, as it uses them: one read per face item where an FP64 product and
+  // The FP32 form's table is rounded to FP32 by the host, with the face scales
+  // multiplied out, as it uses them: one read per face item where an FP64 product and
   // conversions stood (32^3 Taylor-Green 108.6 -> 107.0, 384^2 GLM-MHD 60.7
   // -> 59.8, 128^2 vortex 8.67 -> 8.57).
   constexpr int EPC = cell_elems(ND), GEL = stage_geom_elem(ND, kMFMA), GEOM = stage_geom_len(ND, kMFMA);
@@ -510,7 +510,7 @@ dg_stage_kernel(StageArgs<R> A) {
   const int nE = A.tile_count[tile];
   const int type0 = EPB % EPC ? A.tile_type[tile] : 0;
   const int inst = A.tile_inst ? A.tile_inst[tile] : 0;
-  const double tg = A.geom[(size_t)inst * GEOM + (tid < GEOM ? tid : GEOM - 1)];
+  const R tg = A.geom[(size_t)inst * GEOM + (tid < GEOM ? tid : GEOM - 1)];
   // the instance's switch, parameters and step
   const int on = A.inst_active ? A.inst_active[inst] : 1;
   const Phys phys = Phys::from(A.inst_prm + (size_t)inst * kPrmMax);
@@ -568,7 +568,7 @@ dg_stage_kernel(StageArgs<R> A) {
     const int t = k * S::BLOCK + tid;
     if ((k + 1) * S::BLOCK <= TV || t < TV) reinterpret_cast<TileVec *>(sW)[t] = tq[k];
   }
-  if (tid < GEOM) sG[tid] = R(tg);
+  if (tid < GEOM) sG[tid] = tg;
   if constexpr (kTwo) {
     if (t2 < nitems && it2.job.x >= 0 && (unsigned)(it2.job.y - e0) >= (unsigned)EPB) {
       R *const g = sS + (((it2.job.x >> 7) & 3) * NFP + t2 - small_div<NFP, MAXT>(t2) * NFP) * NCOLS + (it2.job.x & 127) * NC;
