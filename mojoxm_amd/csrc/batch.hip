@@ -95,10 +95,12 @@ using GroupKey = std::tuple<int, int, int, int, int, long long>;  // dim, P, phy
 struct Arena {
   DevBuf<double> qd[3];
   DevBuf<float> qf[3];
-  // limiter (groups with it): cell means [3][slots*NC], node extrema
+  // limiter (groups with it): cell means [3][slots*NC] and node extrema
   // [3][slots*NCL][2] (the limited components: all NC in 3D, component 0 in
-  // 2D) and factors [3][slots] of the stage buffers
-  DevBuf<double> lmean, ltheta, lext;
+  // 2D; in the state's precision) of the stage buffers, and q's factors
+  // [slots], which stage 1 of a step leaves for the others
+  DevBuf<double> lmean, ltheta;
+  DevBuf<char> lext;
   DevBuf<double> geom, iprm, idt, ipost;  // geom, geomf: one table per instance slot
   DevBuf<float> geomf;
   DevBuf<int> conn;  // limiter: partner slot per face
@@ -246,7 +248,8 @@ size_t instance_bytes(const ElemTables &t, int NP, int NC, int NFP, int dim, int
   b += tiles * 3 * sizeof(int);                                     // tile_count, tile_type, tile_inst
   b += (MXM_PRM_MAX + 2) * sizeof(double) + 4 * sizeof(int);        // per-instance scalars
   b += t.geom.size() * sizeof(double) + t.geomf.size() * sizeof(float);
-  if (limiter) b += slots * (3 * NC + 6 * (dim == 3 ? NC : 1) + 3) * sizeof(double);  // means, factors, extrema
+  if (limiter)  // means and factors, extrema
+    b += slots * (3 * NC + 1) * sizeof(double) + slots * 6 * (dim == 3 ? NC : 1) * word;
   return b;
 }
 
@@ -474,11 +477,11 @@ struct Batch {
   // and clears their pending factors (stream order: after the steps
   // enqueued so far)
   void materialize(BGroup &g, int s0, int n) {
-    const size_t S = g.ar.ltheta.n / 3;
+    const size_t S = g.ar.ltheta.n;
     if (n <= 0 || (size_t)s0 + n > S) return;
     auto limit = [&](auto *q) {
-      MXM_HIP(launch_bj_limit(q, g.ar.ltheta.p, g.ar.lmean.p, g.ar.lext.p, g.ar.conn.p, s0, n, g.NP, g.NC, g.NF, g.dim,
-                              g.eps, g.stream));
+      MXM_HIP(launch_bj_limit(q, g.ar.ltheta.p, g.ar.lmean.p, reinterpret_cast<decltype(q)>(g.ar.lext.p), g.ar.conn.p,
+                              s0, n, g.NP, g.NC, g.NF, g.dim, g.eps, g.stream));
     };
     if (g.prec == MXM_PREC_FP64)
       limit(g.ar.qd[0].p);
@@ -543,9 +546,9 @@ struct Batch {
     hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, g.stream, g.ar.ifail.p + sl, 0, 1);
     MXM_HIP(hipGetLastError());
     if (g.limiter) {  // nothing pending on the new state (the range may hold a removed instance's extrema)
-      const size_t n = (size_t)in.ntiles() * g.epb, ncl = g.dim == 3 ? g.NC : 1;
-      MXM_HIP(launch_fill(g.ar.lmean.p + bs * g.NC, (long long)(n * g.NC), 0.0, g.stream));
-      MXM_HIP(launch_fill(g.ar.lext.p + bs * ncl * 2, (long long)(n * ncl * 2), 0.0, g.stream));
+      const size_t n = (size_t)in.ntiles() * g.epb, per = 2 * (g.dim == 3 ? g.NC : 1) * sizeof(R);
+      MXM_HIP(launch_fill(reinterpret_cast<double *>(g.ar.lext.p + bs * per), (long long)(n * per / sizeof(double)),
+                          no_extrema(), g.stream));
     }
     MXM_HIP(hipEventRecord(st.ev, g.stream));
     st.busy = true;
@@ -601,7 +604,7 @@ struct Batch {
   void compact(BGroup &g) {
     drain(g);
     if (g.limiter && g.ar.ltheta.n) {  // the states move with their limiter factors applied
-      materialize(g, 0, (int)(g.ar.ltheta.n / 3));
+      materialize(g, 0, (int)g.ar.ltheta.n);
       drain(g);
     }
     pull_counters(g);
@@ -706,10 +709,10 @@ struct Batch {
     na.ifail.upload(ifl.data(), ifl.size());
     if (g.limiter) {
       na.lmean.alloc(3 * slots * g.NC);
-      na.lext.alloc(3 * 2 * slots * (g.dim == 3 ? g.NC : 1));
-      na.ltheta.alloc(3 * slots);
-      MXM_HIP(launch_fill(na.lmean.p, (long long)na.lmean.n, 0.0, g.stream));
-      MXM_HIP(launch_fill(na.lext.p, (long long)na.lext.n, 0.0, g.stream));
+      na.lext.alloc(3 * 2 * slots * (g.dim == 3 ? g.NC : 1) * (fp32 ? sizeof(float) : sizeof(double)));
+      na.ltheta.alloc(slots);
+      MXM_HIP(launch_fill(reinterpret_cast<double *>(na.lext.p), (long long)(na.lext.n / sizeof(double)), no_extrema(),
+                          g.stream));
       MXM_HIP(launch_fill(na.ltheta.p, (long long)na.ltheta.n, 1.0, g.stream));
     }
     // ---- commit (no more allocations or copies that can fail) ----
@@ -797,11 +800,12 @@ struct Batch {
     a.inst_active = ar.iactive.p;
     a.inst_fail = ar.ifail.p;
     if (g.limiter) {  // as in the solver: outputs' means and extrema, inputs' pending factors
-      const size_t S = ar.ltheta.n / 3, kn = S * g.NC, kx = S * (g.dim == 3 ? g.NC : 1) * 2;
-      a.mean = ar.lmean.p + pl.out * kn, a.ext = ar.lext.p + pl.out * kx;
-      a.lim_mn_in = ar.lmean.p + pl.in * kn, a.lim_ext_in = ar.lext.p + pl.in * kx;
-      a.lim_th_in = ar.ltheta.p + pl.in * S;
-      a.lim_th_a = ar.ltheta.p + pl.qa * S, a.lim_mn_a = ar.lmean.p + pl.qa * kn;
+      const size_t S = ar.ltheta.n, kn = S * g.NC, kx = S * (g.dim == 3 ? g.NC : 1) * 2;
+      R *const ext = reinterpret_cast<R *>(ar.lext.p);
+      a.mean = ar.lmean.p + pl.out * kn, a.ext = ext + pl.out * kx;
+      a.lim_mn_in = ar.lmean.p + pl.in * kn, a.lim_ext_in = ext + pl.in * kx;
+      a.lim_th_in = pl.in == 0 ? ar.ltheta.p : nullptr;
+      a.lim_th_a = ar.ltheta.p, a.lim_mn_a = ar.lmean.p + pl.qa * kn;
       a.conn = ar.conn.p, a.lim_eps2 = g.eps * g.eps;
     }
     a.w = g.w.p;

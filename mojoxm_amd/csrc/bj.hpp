@@ -24,7 +24,8 @@ __device__ __forceinline__ double div_rounded(double n, double d) {
 }
 
 // mean [slots][NC], ext [slots][NCL][2] (NCL = NC with ALL, else component 0
-// only), nb = conn[e] of conn [slots][NF], the partner slot of each face (the
+// only) in the state's precision, whose values they are (NaN: nothing pending,
+// no factor below 1), nb = conn[e] of conn [slots][NF], the partner slot of each face (the
 // element's own on a boundary, which constrains only with ALL)
 template <int NF>
 __device__ __forceinline__ void bj_neighbours(int e, const int *conn, int (&nb)[NF]) {
@@ -32,9 +33,9 @@ __device__ __forceinline__ void bj_neighbours(int e, const int *conn, int (&nb)[
   for (int f = 0; f < NF; ++f) nb[f] = conn[(size_t)e * NF + f];
 }
 // the smaller of th and the factor that component c asks for
-template <int NC, bool ALL, int NF>
+template <int NC, bool ALL, int NF, class R>
 __device__ __forceinline__ double bj_theta_comp(int e, int c, const int (&nb)[NF], const double *mean,
-                                                const double *ext, double eps2, double th) {
+                                                const R *ext, double eps2, double th) {
   constexpr int NCL = ALL ? NC : 1;
   const double bm = mean[(size_t)e * NC + c];
   double mn = bm, mx = bm;
@@ -50,7 +51,7 @@ __device__ __forceinline__ double bj_theta_comp(int e, int c, const int (&nb)[NF
   const double nD = bm - mn < 0.0 ? 0.0 : bm - mn;
 #pragma unroll
   for (int s = 0; s < 2; ++s) {  // the smallest and the largest node value
-    const double d = ext[((size_t)e * NCL + c) * 2 + s] - bm;
+    const double d = double(ext[((size_t)e * NCL + c) * 2 + s]) - bm;
     const double da = d >= 0.0 ? d : -d;
     if (da <= 1.0e-30) continue;
     const double D = d > 0.0 ? pD : nD;
@@ -60,8 +61,8 @@ __device__ __forceinline__ double bj_theta_comp(int e, int c, const int (&nb)[NF
   }
   return th;
 }
-template <int NC, bool ALL, int NF>
-__device__ __forceinline__ double bj_theta(int e, const int (&nb)[NF], const double *mean, const double *ext,
+template <int NC, bool ALL, int NF, class R>
+__device__ __forceinline__ double bj_theta(int e, const int (&nb)[NF], const double *mean, const R *ext,
                                            double eps2) {
   double th = 1.0;
 #pragma unroll

@@ -45,9 +45,9 @@ namespace mxm {
 namespace {
 
 // one thread per element slot
-template <int NC, bool ALL>
+template <class R, int NC, bool ALL>
 __global__ __launch_bounds__(256) void bj_theta_kernel(double *__restrict__ theta, const double *__restrict__ mean,
-                                                       const double *__restrict__ ext, const int *__restrict__ conn,
+                                                       const R *__restrict__ ext, const int *__restrict__ conn,
                                                        int e0, int n, double eps2) {
   constexpr int NF = ALL ? 4 : 3;
   const int i = blockIdx.x * 256 + threadIdx.x;
@@ -57,14 +57,13 @@ __global__ __launch_bounds__(256) void bj_theta_kernel(double *__restrict__ thet
   theta[e0 + i] = bj_theta<NC, ALL, NF>(e0 + i, nb, mean, ext, eps2);
 }
 
-// the limited state written in place, then extrema equal to the means and
-// theta = 1 (a stage takes q_a's theta as it is stored): a block holds whole
+// the limited state written in place, then extrema of NaN and theta = 1 (a stage takes q_a's theta as it is stored): a block holds whole
 // elements, one thread per node, so every node has read theta before the
 // element's first thread resets it
 template <class R, int NC, bool ALL>
 __global__ __launch_bounds__(256) void bj_apply_kernel(R *__restrict__ q, double *__restrict__ theta,
-                                                       const double *__restrict__ mean, double *__restrict__ ext,
-                                                       int e0, int n, int NP) {
+                                                       const double *__restrict__ mean, R *__restrict__ ext, int e0,
+                                                       int n, int NP) {
   constexpr int NCL = ALL ? NC : 1;
   const int epb = 256 / NP;
   const int el = threadIdx.x / NP, node = threadIdx.x - el * NP;
@@ -77,7 +76,7 @@ __global__ __launch_bounds__(256) void bj_apply_kernel(R *__restrict__ q, double
   if (node == 0) {
     theta[e] = 1.0;
 #pragma unroll
-    for (int c = 0; c < NCL; ++c) ext[(e * NCL + c) * 2] = ext[(e * NCL + c) * 2 + 1] = mean[e * NC + c];
+    for (int c = 0; c < NCL; ++c) ext[(e * NCL + c) * 2] = ext[(e * NCL + c) * 2 + 1] = R(__builtin_nan(""));
   }
   if (!(th < 1.0)) return;
   R *qn = q + (e * NP + node) * NC;
@@ -94,9 +93,9 @@ __global__ void fill_kernel(double *p, long long n, double v) {
 }
 
 template <class R, int NC, bool ALL>
-void limit_nc(R *q, double *theta, const double *mean, double *ext, const int *conn, int e0, int n, int NP,
+void limit_nc(R *q, double *theta, const double *mean, R *ext, const int *conn, int e0, int n, int NP,
               double eps2, hipStream_t s) {
-  hipLaunchKernelGGL((bj_theta_kernel<NC, ALL>), dim3((n + 255) / 256), dim3(256), 0, s, theta, mean, ext, conn, e0,
+  hipLaunchKernelGGL((bj_theta_kernel<R, NC, ALL>), dim3((n + 255) / 256), dim3(256), 0, s, theta, mean, ext, conn, e0,
                      n, eps2);
   const int epb = 256 / NP;
   hipLaunchKernelGGL((bj_apply_kernel<R, NC, ALL>), dim3((n + epb - 1) / epb), dim3(256), 0, s, q, theta, mean, ext,
@@ -106,7 +105,7 @@ void limit_nc(R *q, double *theta, const double *mean, double *ext, const int *c
 }  // namespace
 
 template <class R>
-hipError_t launch_bj_limit(R *q, double *theta, const double *mean, double *ext, const int *conn, int e0, int n,
+hipError_t launch_bj_limit(R *q, double *theta, const double *mean, R *ext, const int *conn, int e0, int n,
                            int NP, int NC, int NF, int dim, double eps, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   if (NP > 256 || NF != dim + 1) return hipErrorInvalidValue;
@@ -134,7 +133,7 @@ hipError_t launch_fill(double *p, long long n, double v, hipStream_t s) {
 
 template hipError_t launch_bj_limit<double>(double *, double *, const double *, double *, const int *, int, int, int,
                                             int, int, int, double, hipStream_t);
-template hipError_t launch_bj_limit<float>(float *, double *, const double *, double *, const int *, int, int, int,
+template hipError_t launch_bj_limit<float>(float *, double *, const double *, float *, const int *, int, int, int,
                                            int, int, int, double, hipStream_t);
 
 }  // namespace mxm

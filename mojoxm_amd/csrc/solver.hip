@@ -59,10 +59,12 @@ struct Solver {
   // state trio q, q1, q2: FP64 (MXM_PREC_FP64) or FP32 (MXM_PREC_FP32_MFMA)
   DevBuf<double> q, q1, q2;
   DevBuf<float> f, f1, f2;
-  // limiter: cell means [3][Kd*NC], node extrema [3][Kd*NCL][2] (the limited
-  // components: all NC in 3D, component 0 in 2D) and factors [3][Kd] of the
-  // stage buffers (q, q1, q2)
-  DevBuf<double> lmean, ltheta, lext;
+  // limiter: cell means [3][Kd*NC] and node extrema [3][Kd*NCL][2] (the
+  // limited components: all NC in 3D, component 0 in 2D; in the state's
+  // precision) of the stage buffers (q, q1, q2), and q's factors [Kd], which
+  // stage 1 of a step leaves for the others
+  DevBuf<double> lmean, ltheta;
+  DevBuf<char> lext;
   DevBuf<double> geom, Dt, Lt, w, dprm;
   DevBuf<double> Dn, dpart;  // diagnostics: nodal derivative, tile partials
   PinBuf results;            // diagnostics and speed, written by the kernels
@@ -156,10 +158,14 @@ struct Solver {
 
   // components the limiter bounds
   int ncl() const { return dim == 3 ? NC : 1; }
-  // nothing pending: extrema equal to the means, factors 1
+  // extrema of stage buffer b
+  template <class R>
+  R *extrema(int b) const {
+    return reinterpret_cast<R *>(lext.p) + (size_t)b * Kd * ncl() * 2;
+  }
+  // nothing pending: no extrema, factors 1
   void clear_pending() {
-    MXM_HIP(launch_fill(lmean.p, (long long)lmean.n, 0.0, stream));
-    MXM_HIP(launch_fill(lext.p, (long long)lext.n, 0.0, stream));
+    MXM_HIP(launch_fill(reinterpret_cast<double *>(lext.p), (long long)(lext.n / sizeof(double)), no_extrema(), stream));
     MXM_HIP(launch_fill(ltheta.p, (long long)ltheta.n, 1.0, stream));
   }
   bool has_wide() const { return prec == MXM_PREC_FP32_MFMA && stage_has_wide(dim, NP, NFP, NC); }
@@ -186,8 +192,8 @@ struct Solver {
       }
     }
     lmean.alloc((size_t)3 * Kd * NC);
-    lext.alloc((size_t)3 * 2 * Kd * ncl());
-    ltheta.alloc((size_t)3 * Kd);
+    lext.alloc((size_t)3 * 2 * Kd * ncl() * state_elem_bytes());
+    ltheta.alloc(Kd);
     if (limiter) clear_pending();
     conn.upload(t.conn.data(), t.conn.size());
     maxj = t.fj.maxj;
@@ -270,11 +276,11 @@ struct Solver {
     // extrema; the inputs' pending factors are computed and applied as they
     // are read
     if (limiter) {
-      const size_t kn = (size_t)Kd * NC, kx = (size_t)Kd * ncl() * 2;
-      a.mean = lmean.p + pl.out * kn, a.ext = lext.p + pl.out * kx;
-      a.lim_mn_in = lmean.p + pl.in * kn, a.lim_ext_in = lext.p + pl.in * kx;
-      a.lim_th_in = ltheta.p + (size_t)pl.in * Kd;
-      a.lim_th_a = ltheta.p + (size_t)pl.qa * Kd, a.lim_mn_a = lmean.p + pl.qa * kn;
+      const size_t kn = (size_t)Kd * NC;
+      a.mean = lmean.p + pl.out * kn, a.ext = extrema<R>(pl.out);
+      a.lim_mn_in = lmean.p + pl.in * kn, a.lim_ext_in = extrema<R>(pl.in);
+      a.lim_th_in = pl.in == 0 ? ltheta.p : nullptr;
+      a.lim_th_a = ltheta.p, a.lim_mn_a = lmean.p + pl.qa * kn;  // q_a is q in every stage
       a.conn = conn.p, a.lim_eps2 = eps * eps;
     }
     a.w = w.p;
@@ -292,12 +298,13 @@ struct Solver {
   StageLaunch kernel() const { return limiter ? find(cfg, true) : launch; }
 
   // writes the limited values of stage buffer b (0 = q); nothing is pending
-  // on it afterwards
+  // on it afterwards, nor on q (between a step's stages only q itself may be
+  // given here, since the factors of q are used up)
   void materialize(int b) {
-    const size_t kn = (size_t)Kd * NC, kx = (size_t)Kd * ncl() * 2;
     auto limit = [&](auto *t) {
-      MXM_HIP(launch_bj_limit(t, ltheta.p + (size_t)b * Kd, lmean.p + b * kn, lext.p + b * kx, conn.p, 0, Kd, NP, NC,
-                              NF, dim, eps, stream));
+      MXM_HIP(launch_bj_limit(t, ltheta.p, lmean.p + (size_t)b * Kd * NC,
+                              extrema<std::remove_pointer_t<decltype(t)>>(b), conn.p, 0, Kd, NP, NC, NF, dim, eps,
+                              stream));
     };
     if (prec == MXM_PREC_FP64)
       limit(b == 0 ? q.p : b == 1 ? q1.p : q2.p);

@@ -70,17 +70,18 @@ struct StageArgs {
   const int *inst_active;   // [n_inst] or nullptr (all active)
   int *inst_fail;           // [n_inst] or nullptr: set to 1 when a stored value is not finite
   double *mean;             // [slots][NC] or nullptr: cell means sum_i w_i q_out_i of the stored state
-  double *ext;              // [slots][NCL][2] (with mean): smallest and largest stored node value of the
+  R *ext;                   // [slots][NCL][2] (with mean): smallest and largest stored node value of the
                             // limited components (all NC in 3D, component 0 in 2D)
   const double *w;          // [NP] node weights (with mean)
   // Limiter (mean != nullptr).  The factors pending on q_in are computed
-  // from its means and node extrema as it is read (extrema equal to the means:
-  // nothing pending) and stored; q_a's are those that stage 1 stored.  A value
+  // from its means and node extrema as it is read (NaN extrema: nothing
+  // pending); stage 1 stores those of its input, which is q_a of the others.  A value
   // read from q_in (tile and partner traces) or q_a is used as
   // mean + theta (q - mean) where its element's theta < 1, which is the state
   // the limiter would have stored.
-  const double *lim_mn_in, *lim_ext_in;  // q_in: means [slots][NC], extrema [slots][NCL][2]
-  double *lim_th_in;                     // q_in: theta [slots], written for the tile's elements
+  const double *lim_mn_in;               // q_in: means [slots][NC]
+  const R *lim_ext_in;                   // q_in: extrema [slots][NCL][2]
+  double *lim_th_in;                     // q_in: theta [slots], written for the tile's elements, or nullptr
   const double *lim_th_a, *lim_mn_a;     // q_a: theta, means
   const int *conn;                       // [slots][NF] partner slot of each face
   double lim_eps2;                       // Venkatakrishnan's eps^2
@@ -605,7 +606,7 @@ dg_stage_kernel(StageArgs<R> A) {
       if (theta) {
         const double th = bj_theta<NC, ND == 3, NF>(the, thnb, A.lim_mn_in, A.lim_ext_in, A.lim_eps2);
         sTh[tid] = th;
-        if (thj < 0) A.lim_th_in[the] = th;
+        if (thj < 0 && A.lim_th_in) A.lim_th_in[the] = th;
       }
       for (int i = tid + S::BLOCK; i < EPB + A.maxj; i += S::BLOCK) {  // more jobs than threads left
         const int2 job = jobs[i - EPB];
@@ -619,7 +620,7 @@ dg_stage_kernel(StageArgs<R> A) {
   // the q_in tile's pending limiter factors, applied in place to the
   // values this thread stored
   if constexpr (LIM) {
-    if (kThetaComp && tid < EPB) A.lim_th_in[e0 + tid] = sTh[tid];
+    if (kThetaComp && tid < EPB && A.lim_th_in) A.lim_th_in[e0 + tid] = sTh[tid];
 #pragma unroll
     for (int k = 0; k < QPT; ++k) {
       const int t = k * S::BLOCK + tid;
@@ -1084,8 +1085,8 @@ dg_stage_kernel(StageArgs<R> A) {
           lo = v < lo ? v : lo;
           hi = v > hi ? v : hi;
         }
-        A.ext[((size_t)(e0 + el) * NCL + c) * 2] = lo;
-        A.ext[((size_t)(e0 + el) * NCL + c) * 2 + 1] = hi;
+        A.ext[((size_t)(e0 + el) * NCL + c) * 2] = R(lo);
+        A.ext[((size_t)(e0 + el) * NCL + c) * 2 + 1] = R(hi);
       }
     }
   }
