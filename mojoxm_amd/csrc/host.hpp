@@ -78,8 +78,14 @@ struct Tiling {
   int slots() const { return ntiles * epb; }
 };
 // room: the most tiles that blocks cut off at the mesh's edge may make.
-// Alone on the device, one tile per CU; one of many, few, so that small
-// meshes of about the same size still take equal ranges of tiles.
+// Alone on the device, one tile per CU (build_tiling has the times).  One of
+// many shares the CUs, and every tile counts: us per stage of a batch, room 16
+// / 256: 48 Euler meshes of 17 to 35 squares, P = 3, FP32 16.7 / 17.4, FP64
+// 23.7 / 24.2, 48 of 3 to 6 cubes 24.3 / 25.8 and 36.1 / 37.5.  No room at all
+// is faster still for the smallest (64 of 9 to 17 squares 8.9 -> 8.2 us, others
+// within 2 %), but there meshes of nearly the same size would no longer take
+// equal ranges of tiles, which is what lets one take the place of another in
+// an arena without a compaction.
 constexpr int kRoomAlone = 256, kRoomBatch = 16;
 Tiling build_tiling(const HostMesh &m, int epb, int NFP, int room);
 

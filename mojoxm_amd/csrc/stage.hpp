@@ -141,8 +141,9 @@ constexpr int kStageCfgMax = 4;
 // elements -- until the block's LDS at FP64 (the operand array -- the q_in
 // tile and the face fluxes, later the ND*NP flux planes, rows of
 // EPB*NC + 1 values -- and 8 bytes for each invJ entry and volume of the
-// elements, an allowance for the geometry) fits 64 KB, which only the
-// two-fluid state (NC = 17) needs.  Tiles are blocks of cells, so the LDS
+// elements, an allowance for the geometry table and the limiter's arrays,
+// which are of about that size; the kernel asserts its own sum) fits 64 KB,
+// which only the two-fluid state (NC = 17) and, at P = 1, MHD (NC = 9) need.  Tiles are blocks of cells, so the LDS
 // is sized for what a tile can hold; the host builds the tiles with the
 // same value.
 //
@@ -427,6 +428,7 @@ dg_stage_kernel(StageArgs<R> A) {
   // has more slots than threads (28^3 Euler 66 / 57.6 / 59.2).
   constexpr bool kThetaComp = LIM && ND == 3 && NC > 1 && EPB * (1 + NF) <= S::BLOCK;
   static_assert(!kThetaComp || EPB * (1 + NF) * (1 + NF) * sizeof(int) <= NFF * NCOLS * sizeof(R), "slots' neighbours");
+  static_assert(sizeof(sB) + sizeof(sG) + sizeof(sMap) + sizeof(sLim) + sizeof(sTh) <= 65536, "LDS of a block");
   R *const sW = sB;
   R *const sS = sB + TILE;
   [[maybe_unused]] int *const sNb = reinterpret_cast<int *>(sS);  // [slot][1 + NF] (kThetaComp)
@@ -706,8 +708,8 @@ dg_stage_kernel(StageArgs<R> A) {
 
   // ---- 2b. nodal flux of the own node, and the RK terms of q_in ----------
   // qa becomes a q_a + b q_in + c dt S(q_in) (FP64); the flux, mapped to
-  // reference directions by invJ in FP64, waits in registers until every
-  // read of the q_in tile is done.
+  // reference directions by invJ in the form's own precision, waits in
+  // registers until every read of the q_in tile is done.
   R Fk[ND * NC];
   double qa[NC];
   if constexpr (kQaLate) {
@@ -762,6 +764,9 @@ dg_stage_kernel(StageArgs<R> A) {
   // blocks per CU (us per stage: 32^3 Taylor-Green 115 -> 108, 19^3 30.7 ->
   // 29.3, 113^2 P = 4 Maxwell 11.3 -> 11.0, 128^2 vortex 8.8 -> 8.6).
   constexpr int KL = (KPAD - KVP) / 4, KD = KVP / 4;      // k-steps of the lift and volume products
+  // Up to 30 entries a lane (3D P = 3); the 81 of P = 4 would take the registers
+  // of other blocks (13^3 Euler 27.6 us loaded as it goes, 38.3 ahead, shallow
+  // water 21.5 and 29.6).
   constexpr bool kAhead = kMFMA && MT * (KL > KD ? KL : KD) <= 32;
   constexpr int WAVES = S::BLOCK / 64, NTW = (NT + WAVES - 1) / WAVES;  // column tiles per wave
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

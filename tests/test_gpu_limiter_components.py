@@ -1,4 +1,4 @@
-"""3D limiter, whose factor is the minimum over all components: every order
+"""The 3D limiter, whose factor is the minimum over all components: every order
 and every number of components, on meshes of several ragged tiles with
 boundaries (neighbours that are the element itself) and without, against the
 oracle in both forms (the bars of the limited parity tests: 1e-12, FP32
@@ -54,3 +54,34 @@ def test_limited_components(oracle, name, P, precision):
         om = oracle.Mesh(3, P, n, L, list(bc) if bc else None)
         want = om.step(phys.phys_id, phys.params(), q, dt, 2, limiter=True, eps=0.1)
         assert rel_l2(got, want) < (TOL if precision == M.PREC_FP64 else TOL32)
+
+
+PHYS_2D = {
+    "euler": ph.Euler(flux_type=ph.FLUX_HLLE),
+    "sw": ph.ShallowWater2D(hll=True),
+    "maxwell": ph.Maxwell2D(),
+    "glm": ph.MHDGLM2D(c_h=1.3, alpha_d=1.3 / 0.18),
+}
+MESHES_2D = [((17, 9), None), ((13, 11), (2, 2, 1, 1)), ((1, 1), None)]
+
+
+@pytest.mark.parametrize("P", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("name", list(PHYS_2D))
+def test_limited_triangles_fp32(oracle, name, P):
+    """The FP32 form on triangles (one limited component) against the oracle:
+    ragged tiles, boundaries, every order."""
+    phys, L = PHYS_2D[name], (1.0, 0.8)
+    for n, bc in MESHES_2D:
+        print(name, P, n, bc, flush=True)
+        bcs = M.BoundaryConditions2D(*bc) if bc else None
+        dt = 0.05 * min(L) / max(n) / (2 * P + 1)
+        with M.Solver(n, L, phys, P=P, bcs=bcs, precision=M.PREC_FP32_MFMA) as s:
+            q = random_state(phys, s.num_elements, s.NP, np.random.default_rng(P), 2)
+            q = q.astype(np.float32).astype(np.float64)
+            s.enable_cell_limiter(True, 0.1)
+            s.set_state(q)
+            s.step_ssprk3(dt, 2)
+            got = s.get_state()
+        om = oracle.Mesh(2, P, n, L, list(bc) if bc else None)
+        want = om.step(phys.phys_id, phys.params(), q, dt, 2, limiter=True, eps=0.1)
+        assert rel_l2(got, want) < TOL32
