@@ -1075,16 +1075,20 @@ dg_stage_kernel(StageArgs<R> A) {
   // sum_i w_i q_i per (element, component) in node order, FP64, from the
   // stored values: what a separate pass over q_out would compute
   if constexpr (LIM) {
+    // 35 and 56 nodes are not read all at once: Maxwell's FP64 kernel at P = 5
+    // held 132 VGPRs for that, 3 waves per SIMD where its LDS lets 4 run (15^3
+    // limited, us per stage: 242.7, 116 VGPRs 218.3)
+    constexpr int kUnroll = NP > 20 ? 8 : NP;
     for (int p = tid; p < nE * NC; p += S::BLOCK) {
       const int el = p / NC, c = p - el * NC;
       double sm = 0.0;
-#pragma unroll
+#pragma unroll kUnroll
       for (int n = 0; n < NP; ++n) sm += A.w[n] * double(sW[(el * NP + n) * NC + c]);
       A.mean[(size_t)(e0 + el) * NC + c] = sm;
       constexpr int NCL = ND == 3 ? NC : 1;  // the components the limiter bounds
       if (c < NCL) {
         double lo = double(sW[el * NP * NC + c]), hi = lo;
-#pragma unroll
+#pragma unroll kUnroll
         for (int n = 1; n < NP; ++n) {
           const double v = double(sW[(el * NP + n) * NC + c]);
           lo = v < lo ? v : lo;
