@@ -819,7 +819,10 @@ dg_stage_kernel(StageArgs<R> A) {
   // stands before the next rows are asked for.  Against one set, loaded and
   // waited for, us per stage: 512^2 vortex 149.7 -> 145.4, 128^2 14.1 -> 13.7,
   // 32^3 Taylor-Green 181 -> 176.5, 16^3 P = 2 advection 7.5 -> 6.7.
-  // A set holds up to 16 entries, and two rows of 9 or 10 where the product
+  // A set holds up to 16 entries; three rows of 3, since five (two sets of 30
+  // scalar registers) gained nothing at best and made larger meshes slower (us
+  // per stage, five rows / three: 320^2 P = 3 advection 22.1 / 19.0, limited
+  // 36.9 / 31.2, 34^3 P = 2 34.0 / 31.6); and two rows of 9 or 10 where the product
   // is longer than a 2D P = 3 one (20 rows): with one row of 10 a wave had 10
   // FMAs to cover each wait (us per stage, one set / one row / two rows:
   // 18^3 P = 3 Maxwell 51.4 / 58.3 / 49.1, MHD 71.5 / 81.5 / 66.9, 13^3 P = 4
@@ -839,7 +842,7 @@ dg_stage_kernel(StageArgs<R> A) {
       }
       return;
     }
-    constexpr int RB = IH <= 8 ? 16 / IH : IH <= 10 && N > 20 ? 2 : 1, SETS = (N + RB - 1) / RB;
+    constexpr int RB = IH == 3 ? 3 : IH <= 8 ? 16 / IH : IH <= 10 && N > 20 ? 2 : 1, SETS = (N + RB - 1) / RB;
     double o[2][RB][IH], v[2][RB];
     auto load = [&](int b, int s) {
 #pragma unroll
