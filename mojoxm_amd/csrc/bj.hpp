@@ -2,7 +2,7 @@
 // smoothing, from the cell means of the element and its face neighbours and
 // the element's smallest and largest node value (limiter.hip says why those
 // suffice).  The stage kernels compute it for the elements they read; the
-// theta kernel computes the same bits for readers of a stored state.
+// limiter's own kernel computes the same bits for readers of a stored state.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -1,8 +1,8 @@
 // limiter.hpp -- the Barth-Jespersen limiter of a stored state.  The stage
 // kernel writes the cell means and node extrema of what it stores
 // (StageArgs::mean, StageArgs::ext); the next stage kernel computes the
-// factors from them and applies them as it reads (StageArgs::lim_*).  These
-// kernels do the same for every other reader of the state.
+// factors from them and applies them as it reads (StageArgs::lim_*).  This
+// does the same for every other reader of the state.
 #pragma once
 #include <hip/hip_runtime.h>
 
