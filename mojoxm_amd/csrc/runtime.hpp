@@ -86,26 +86,6 @@ struct DevBuf {
   size_t bytes() const { return n * sizeof(T); }
 };
 
-// Pinned host memory for a few results that kernels write themselves; the
-// host reads it after it has waited for the stream.
-struct PinBuf {
-  double *p = nullptr;
-  size_t n = 0;
-  PinBuf() = default;
-  PinBuf(const PinBuf &) = delete;
-  PinBuf &operator=(const PinBuf &) = delete;
-  ~PinBuf() {
-    if (p) (void)hipHostFree(p);
-  }
-  void reserve(size_t count) {
-    if (count <= n) return;
-    if (p) (void)hipHostFree(p);
-    p = nullptr, n = 0;
-    MXM_HIP(hipHostMalloc(reinterpret_cast<void **>(&p), count * sizeof(double)));
-    n = count;
-  }
-};
-
 // A captured step sequence: the graph and its executable live and die
 // together (a profiler or the runtime may still refer to the graph's nodes
 // while the executable is launched).

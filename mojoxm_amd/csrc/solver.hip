@@ -67,7 +67,7 @@ struct Solver {
   DevBuf<char> lext;
   DevBuf<double> geom, Dt, Lt, w, dprm;
   DevBuf<double> Dn, dpart;  // diagnostics: nodal derivative, tile partials
-  PinBuf results;            // diagnostics and speed, written by the kernels
+  DevBuf<double> dout;       // their results where there is no pinned memory (collect)
   DevBuf<float> geomf, Aop;  // geomf: the FP32 stage kernel's (ElemTables)
   DevBuf<int> conn;  // limiter: partner slot per face
   DevBuf<int> fmap, tile_count, tile_type;
@@ -392,17 +392,37 @@ struct Solver {
     return cfg;
   }
 
+  // h[0..n) = what the kernels that run(out) enqueues write to out: pinned
+  // host memory, so that one wait brings it, or device memory and a copy
+  template <class F>
+  void collect(size_t n, double *h, F &&run) {
+    static_assert(PinnedPool::kPiece >= (3 * kDiagMaxNC + 2) * sizeof(double), "results fit a piece");
+    const PinnedPiece piece;
+    double *out = reinterpret_cast<double *>(piece.p);
+    if (!piece.pinned) {
+      if (dout.n < n) dout.alloc(n);
+      out = dout.p;
+    }
+    run(out);
+    if (!piece.pinned) MXM_HIP(hipMemcpyAsync(h, out, n * sizeof(double), hipMemcpyDeviceToHost, stream));
+    MXM_HIP(hipStreamSynchronize(stream));
+    if (piece.pinned) std::memcpy(h, out, n * sizeof(double));
+  }
+
   // int q_c, int q_c^2, max |q_c|, KE, enstrophy of the current state
   // (3*NC + 2 values; NaN for KE and enstrophy without a velocity)
   void diagnostics(double *h) {
     const size_t per = (size_t)kDiagSums * 2 + kDiagMaxNC;
     if (dpart.n < (size_t)ntiles * per) dpart.alloc((size_t)ntiles * per);
-    results.reserve(3 * NC + 2);
+    collect(3 * NC + 2, h, [&](double *out) { enqueue_diagnostics(out); });
+    if (!diag_nvel(phys)) h[3 * NC] = h[3 * NC + 1] = std::nan("");
+  }
+  void enqueue_diagnostics(double *out) {
     auto fill = [&](auto &a) {
       a.cell = geom.p + geom.n - cell_geom_len(dim), a.tile_type = tile_type.p;
       a.w = w.p, a.Dn = Dn.p, a.tile_count = tile_count.p;
       a.epb = til.epb, a.tile0 = 0, a.ntiles = ntiles, a.NC = NC, a.nvel = diag_nvel(phys);
-      a.part = dpart.p, a.pmax = dpart.p + (size_t)ntiles * kDiagSums * 2, a.out = results.p;
+      a.part = dpart.p, a.pmax = dpart.p + (size_t)ntiles * kDiagSums * 2, a.out = out;
     };
     if (prec == MXM_PREC_FP64) {
       DiagArgs<double> a{};
@@ -415,9 +435,6 @@ struct Solver {
       fill(a);
       MXM_HIP(launch_diagnostics(dim, P, false, &a, stream));
     }
-    MXM_HIP(hipStreamSynchronize(stream));
-    std::memcpy(h, results.p, (3 * NC + 2) * sizeof(double));
-    if (!diag_nvel(phys)) h[3 * NC] = h[3 * NC + 1] = std::nan("");
   }
 
   // enqueues the largest-signal-speed reduction of the current state on
@@ -444,10 +461,9 @@ struct Solver {
   // the largest signal speed over the nodes of the current state
   double max_wave_speed() {
     if (dpart.n < (size_t)ntiles) dpart.alloc(ntiles);
-    results.reserve(3 * NC + 2);  // once for the diagnostics too: pinning took 26 us of their first call
-    enqueue_max_speed(dpart.p, results.p);
-    MXM_HIP(hipStreamSynchronize(stream));
-    return results.p[0];
+    double speed = 0.0;
+    collect(1, &speed, [&](double *out) { enqueue_max_speed(dpart.p, out); });
+    return speed;
   }
 
   // whether the graphs are those of the present settings and this dt

@@ -3,7 +3,8 @@
 //
 // The state moves in pieces through pinned host buffers: several host threads
 // take pieces in turn, and each has the DMA of its next piece in flight while
-// it permutes and converts the present one.  One pageable copy of the whole
+// it permutes and converts the present one; a state of one piece takes one
+// copy and one wait.  One pageable copy of the whole
 // state and one thread's loop over its elements, into pages that the caller
 // had not touched yet, moved 3 to 5 GB/s of the caller's array.  Reading the
 // 512^2 vortex's 210 MB: FP32 45 -> 4.4 ms, FP64 72 -> 7.4; the 128^2 one's
@@ -16,37 +17,95 @@
 #include <atomic>
 #include <cstdint>
 #include <cstdlib>
+#include <mutex>
 #include <thread>
 #include <vector>
 
 namespace mxm {
 
-// Pinned buffers of the transfers of one solver or batch, kept between them
-// (pageable ones where no pinned memory can be had: the copies then wait).
-struct HostPieces {
+// Pinned buffers of one piece each, shared by every solver and batch of the
+// process: a transfer takes what it needs and gives it back when it ends.  At
+// most kKept are kept for the next one, and none once the last object that
+// may use them is gone.  Pinning memory takes 0.1 to 1 ms at first, which a
+// buffer per object paid for each of them (and held for its life).
+class PinnedPool {
+ public:
   static constexpr size_t kPiece = 1 << 20;  // bytes of device state per piece
-  static constexpr int kThreads = 8;         // at most; each has two pieces
-  char *p = nullptr;
-  size_t size = 0;
-  bool pinned = false;
+  static constexpr int kKept = 16;
+  static PinnedPool &get() {
+    static PinnedPool *pool = new PinnedPool;  // outlives every static object
+    return *pool;
+  }
+  // nullptr where no pinned memory can be had
+  char *take() {
+    {
+      std::lock_guard<std::mutex> l(m_);
+      if (n_ > 0) return free_[--n_];
+    }
+    char *p = nullptr;
+    if (hipHostMalloc(reinterpret_cast<void **>(&p), kPiece) == hipSuccess) return p;
+    (void)hipGetLastError();  // handled by the caller, not the next launch's error
+    return nullptr;
+  }
+  void give(char *p) {
+    {
+      std::lock_guard<std::mutex> l(m_);
+      if (users_ > 0 && n_ < kKept) {
+        free_[n_++] = p;
+        return;
+      }
+    }
+    (void)hipHostFree(p);
+  }
+  void join() {
+    std::lock_guard<std::mutex> l(m_);
+    ++users_;
+  }
+  void leave() {
+    std::lock_guard<std::mutex> l(m_);
+    if (--users_ > 0) return;
+    while (n_ > 0) (void)hipHostFree(free_[--n_]);
+  }
+
+ private:
+  PinnedPool() = default;
+  std::mutex m_;
+  char *free_[kKept] = {};
+  int n_ = 0, users_ = 0;
+};
+
+// One buffer of the pool while it is used; pageable where the pool has none
+// (copies then wait), empty where there is no memory at all.
+struct PinnedPiece {
+  char *p = PinnedPool::get().take();
+  bool pinned = p != nullptr;
+  PinnedPiece() {
+    if (!pinned) p = static_cast<char *>(std::malloc(PinnedPool::kPiece));
+  }
+  PinnedPiece(const PinnedPiece &) = delete;
+  PinnedPiece &operator=(const PinnedPiece &) = delete;
+  ~PinnedPiece() {
+    if (pinned)
+      PinnedPool::get().give(p);
+    else
+      std::free(p);
+  }
+};
+
+// What the transfers of one solver or batch keep between them.
+struct HostPieces {
+  static constexpr size_t kPiece = PinnedPool::kPiece;
+  static constexpr int kThreads = 8;  // at most; each has two pieces
   hipEvent_t ev[2 * kThreads] = {};
-  HostPieces() = default;
+  HostPieces() { PinnedPool::get().join(); }
   HostPieces(const HostPieces &) = delete;
   HostPieces &operator=(const HostPieces &) = delete;
   ~HostPieces() {
     for (auto e : ev)
       if (e) (void)hipEventDestroy(e);
-    release();
+    PinnedPool::get().leave();
   }
-  void release() {
-    if (p && pinned)
-      (void)hipHostFree(p);
-    else
-      std::free(p);
-    p = nullptr, size = 0;
-  }
-  // n buffers, of `bytes` in all
-  hipError_t reserve(int n, size_t bytes) {
+  hipError_t events(int n) {
     for (int k = 0; k < n; ++k) {
       if (ev[k]) continue;
       const hipError_t e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
@@ -55,16 +114,6 @@ struct HostPieces {
         return e;
       }
     }
-    if (bytes <= size) return hipSuccess;
-    bytes = std::max(bytes, std::min(2 * size, 2 * kThreads * kPiece));
-    release();
-    pinned = hipHostMalloc(reinterpret_cast<void **>(&p), bytes) == hipSuccess;
-    if (!pinned) {
-      (void)hipGetLastError();  // handled here, not the next launch's error
-      p = static_cast<char *>(std::malloc(bytes));
-      if (!p) return hipErrorOutOfMemory;
-    }
-    size = bytes;
     return hipSuccess;
   }
 };
@@ -93,15 +142,49 @@ hipError_t move_state(HostPieces &hp, R *dev, const int32_t *ref_of, int slots, 
   if ((size_t)per * node * sizeof(R) > HostPieces::kPiece) return hipErrorInvalidValue;
   const int pieces = (slots + per - 1) / per;
   if (pieces == 0) return hipStreamSynchronize(stream);
+  // slots [begin, begin + n) between a piece and the caller's array
+  auto elements = [&](int begin, int n, R *b) {
+    for (int k = 0; k < n; ++k) {
+      const int el = ref_of[begin + k];
+      R *d = b + (size_t)k * node;
+      if (el < 0) {
+        if (!TO_HOST) std::fill(d, d + node, R(0));
+        continue;
+      }
+      auto *u = h + (size_t)el * node;
+      for (size_t v = 0; v < node; ++v) {
+        if constexpr (TO_HOST)
+          u[v] = double(d[v]);
+        else
+          d[v] = R(u[v]);
+      }
+    }
+  };
+  auto copy = [&](R *b, int begin, int n) {
+    R *const d = dev + (size_t)begin * node;
+    const size_t bytes = (size_t)n * node * sizeof(R);
+    return TO_HOST ? hipMemcpyAsync(b, d, bytes, hipMemcpyDeviceToHost, stream)
+                   : hipMemcpyAsync(d, b, bytes, hipMemcpyHostToDevice, stream);
+  };
+  if (pieces == 1) {  // nothing to overlap: one copy and one wait
+    const PinnedPiece piece;
+    if (!piece.p) return hipErrorOutOfMemory;
+    R *const b = reinterpret_cast<R *>(piece.p);
+    if (!TO_HOST) elements(0, slots, b);
+    const hipError_t c = copy(b, 0, slots), w = hipStreamSynchronize(stream);
+    if (c != hipSuccess || w != hipSuccess) return c != hipSuccess ? c : w;
+    if (TO_HOST) elements(0, slots, b);
+    return hipSuccess;
+  }
   // a thread pays from about two pieces on
   const int threads = std::max(1, std::min({HostPieces::kThreads, pieces / 2, (int)std::thread::hardware_concurrency()}));
   const int ring = pieces > threads ? 2 : 1;  // pieces each thread has under way
   const OnDevice on(device);
-  // a small state takes what it needs: pinning a whole piece for it cost its
-  // first transfer 40 to 50 us (5^3 Euler, P = 2)
-  const size_t stride = ((size_t)std::min(per, slots) * node * sizeof(R) + 255) / 256 * 256;
-  hipError_t e = hp.reserve(threads * ring, (size_t)threads * ring * stride);
+  hipError_t e = hp.events(threads * ring);
   if (e != hipSuccess) return e;
+  const std::vector<PinnedPiece> buffers(threads * ring);
+  for (const PinnedPiece &b : buffers)
+    if (!b.p) return hipErrorOutOfMemory;
   std::atomic<int> next{0}, error{(int)hipSuccess};
   auto work = [&](int t) {
     auto ok = [&](hipError_t r) {
@@ -111,25 +194,8 @@ hipError_t move_state(HostPieces &hp, R *dev, const int32_t *ref_of, int slots, 
     if (t > 0 && !ok(hipSetDevice(device))) return;
     auto begin = [&](int c) { return c * per; };
     auto count = [&](int c) { return std::min(per, slots - c * per); };
-    auto buf = [&](int s) { return reinterpret_cast<R *>(hp.p + (size_t)(t * ring + s) * stride); };
+    auto buf = [&](int s) { return reinterpret_cast<R *>(buffers[t * ring + s].p); };
     int piece[2] = {-1, -1};
-    auto elements = [&](int c, R *b) {
-      for (int k = 0; k < count(c); ++k) {
-        const int el = ref_of[begin(c) + k];
-        R *d = b + (size_t)k * node;
-        if (el < 0) {
-          if (!TO_HOST) std::fill(d, d + node, R(0));
-          continue;
-        }
-        auto *u = h + (size_t)el * node;
-        for (size_t v = 0; v < node; ++v) {
-          if constexpr (TO_HOST)
-            u[v] = double(d[v]);
-          else
-            d[v] = R(u[v]);
-        }
-      }
-    };
     // the buffers in turn: wait for what is under way in one, finish it, put
     // the next piece under way
     bool more = true;
@@ -137,7 +203,7 @@ hipError_t move_state(HostPieces &hp, R *dev, const int32_t *ref_of, int slots, 
       const int at = t * ring + s;
       if (piece[s] >= 0) {
         if (!ok(hipEventSynchronize(hp.ev[at]))) return;
-        if (TO_HOST) elements(piece[s], buf(s));
+        if (TO_HOST) elements(begin(piece[s]), count(piece[s]), buf(s));
         piece[s] = -1;
       }
       int c = more ? next.fetch_add(1) : pieces;
@@ -147,13 +213,8 @@ hipError_t move_state(HostPieces &hp, R *dev, const int32_t *ref_of, int slots, 
         continue;
       }
       idle = 0;
-      if (!TO_HOST) elements(c, buf(s));
-      R *d = dev + (size_t)begin(c) * node;
-      const size_t bytes = (size_t)count(c) * node * sizeof(R);
-      if (!ok(TO_HOST ? hipMemcpyAsync(buf(s), d, bytes, hipMemcpyDeviceToHost, stream)
-                      : hipMemcpyAsync(d, buf(s), bytes, hipMemcpyHostToDevice, stream)) ||
-          !ok(hipEventRecord(hp.ev[at], stream)))
-        return;
+      if (!TO_HOST) elements(begin(c), count(c), buf(s));
+      if (!ok(copy(buf(s), begin(c), count(c))) || !ok(hipEventRecord(hp.ev[at], stream))) return;
       piece[s] = c;
     }
   };

@@ -12,6 +12,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 HIP = r"""
 #pragma once
+#include <atomic>
 #include <condition_variable>
 #include <chrono>
 #include <cstddef>
@@ -70,16 +71,15 @@ struct Event { int device; Stream *s = nullptr; long at = 0; };
 typedef Event *hipEvent_t;
 inline thread_local int cur_device = 0;
 inline hipError_t last_error = hipSuccess;
-inline int fail_events = 0, fail_pinned = 0, fail_copy = 0, live_events = 0, live_pinned = 0;
-inline size_t pinned_bytes = 0;
+inline int fail_events = 0, fail_pinned = 0, fail_copy = 0, live_events = 0, made_pinned = 0;
+inline std::atomic<int> live_pinned{0};
 inline hipError_t bad(hipError_t e) { return last_error = e; }
 inline hipError_t hipGetLastError() { auto e = last_error; last_error = hipSuccess; return e; }
 inline hipError_t hipGetDevice(int *d) { *d = cur_device; return hipSuccess; }
 inline hipError_t hipSetDevice(int d) { cur_device = d; return hipSuccess; }
 inline hipError_t hipHostMalloc(void **p, size_t n) {
   if (fail_pinned > 0) { --fail_pinned; return bad(hipErrorOutOfMemory); }
-  ++live_pinned;
-  pinned_bytes = n;
+  ++live_pinned, ++made_pinned;
   *p = std::malloc(n);
   return hipSuccess;
 }
@@ -165,11 +165,38 @@ int main(int argc, char **argv) {
   const std::string what = argv[1];
   Stream st(0);
   if (what == "sizes") return sizes<double>(st) || sizes<float>(st);
-  if (what == "small") {  // a small state pins what it needs, not whole pieces
-    HostPieces hp;
-    CHECK(!both_ways<float>(hp, 24, 50, 0, &st));
-    CHECK(pinned_bytes <= 2 * 24 * 50 * sizeof(float));
-    CHECK(!both_ways<double>(hp, 5000, 50, 0, &st));  // and grows
+  if (what == "pool") {  // buffers are shared, bounded, and gone with the last object
+    {
+      HostPieces a;
+      CHECK(!both_ways<float>(a, 24, 50, 0, &st));
+      CHECK(made_pinned == 1 && live_events == 0);  // one piece: one buffer, no events
+      {
+        HostPieces b;
+        CHECK(!both_ways<float>(b, 24, 50, 0, &st) && !both_ways<double>(a, 30, 50, 0, &st));
+        CHECK(made_pinned == 1);
+      }
+      CHECK(!both_ways<double>(a, 60000, 50, 0, &st));
+      CHECK(live_pinned <= PinnedPool::kKept);
+      const int made = made_pinned;
+      CHECK(!both_ways<double>(a, 60000, 50, 0, &st));
+      CHECK(made_pinned == made);
+      std::vector<PinnedPiece> many(3 * PinnedPool::kKept);
+      CHECK(live_pinned == 3 * PinnedPool::kKept);
+      many.clear();
+      CHECK(live_pinned == PinnedPool::kKept);
+    }
+    CHECK(live_pinned == 0 && live_events == 0);
+    // several objects, streams and threads at once
+    std::vector<std::thread> t;
+    std::atomic<int> bad{0};
+    for (int k = 0; k < 6; ++k)
+      t.emplace_back([&bad, k] {
+        Stream mine(0);
+        HostPieces hp;
+        for (int r = 0; r < 4; ++r) bad += both_ways<float>(hp, 3000 * (k + 1) + r, 50, 0, &mine);
+      });
+    for (auto &x : t) x.join();
+    CHECK(!bad && live_pinned == 0);
   }
   if (what == "events") {  // a call that could not get its events fails; the next one works
     for (int k = 1; k <= 3; ++k) {
@@ -232,7 +259,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["sizes", "events", "pinned", "device", "small", "copy"])
+@pytest.mark.parametrize("what", ["sizes", "events", "pinned", "device", "pool", "copy"])
 def test_transfer(program, what):
     r = subprocess.run([program, what], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
