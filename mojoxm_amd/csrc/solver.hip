@@ -163,10 +163,18 @@ struct Solver {
   R *extrema(int b) const {
     return reinterpret_cast<R *>(lext.p) + (size_t)b * Kd * ncl() * 2;
   }
-  // nothing pending: no extrema, factors 1
+  // The limiter's buffers are consistent between calls: nothing is pending on
+  // q and its factors are 1 (materialize).  They are not while `stale`: before
+  // their first use, and when stages ran or a state came with the limiter off.
+  bool stale = true;
+  // nothing pending on any stage buffer
   void clear_pending() {
     MXM_HIP(launch_fill(reinterpret_cast<double *>(lext.p), (long long)(lext.n / sizeof(double)), no_extrema(), stream));
+  }
+  void clear_limiter() {
+    clear_pending();
     MXM_HIP(launch_fill(ltheta.p, (long long)ltheta.n, 1.0, stream));
+    stale = false;
   }
   bool has_wide() const { return prec == MXM_PREC_FP32_MFMA && stage_has_wide(dim, NP, NFP, NC); }
   StageLaunch find(int c, bool lim) const { return find_stage(dim, phys, variant, P, prec, c, lim, wide); }
@@ -194,7 +202,8 @@ struct Solver {
     lmean.alloc((size_t)3 * Kd * NC);
     lext.alloc((size_t)3 * 2 * Kd * ncl() * state_elem_bytes());
     ltheta.alloc(Kd);
-    if (limiter) clear_pending();
+    stale = true;
+    if (limiter) clear_limiter();
     conn.upload(t.conn.data(), t.conn.size());
     maxj = t.fj.maxj;
     tile_count.upload(til.count.data(), til.count.size());
@@ -248,6 +257,7 @@ struct Solver {
 
   // Shu-Osher plan of src/ssprk3.mojo:41-78 (FP64 coefficients).
   void stage(int s, double dt) {
+    if (!limiter) stale = true;
     if (prec == MXM_PREC_FP64)
       stage_with(s, dt, q.p, q1.p, q2.p);
     else
@@ -327,11 +337,13 @@ struct Solver {
     const int c0 = cfg;
     try {
       const double t = time_configs(dt, reps, us);
+      if (limiter) clear_limiter();  // of the steps that were timed
       upload_state(h.data());
       return t;
     } catch (...) {
       cfg = c0;
       launch = find(cfg, false);
+      if (limiter) clear_limiter();
       upload_state(h.data());
       throw;
     }
@@ -485,6 +497,7 @@ struct Solver {
   void replay(double dt, int n) {
     if (n <= 0) return;
     prepare(dt, n);
+    if (!limiter) stale = true;
     for (; n >= kGraphSteps; n -= kGraphSteps) MXM_HIP(hipGraphLaunch(gfull.exec, stream));
     if (n) MXM_HIP(hipGraphLaunch(grem[n].exec, stream));
     if (limiter) materialize(0);
@@ -510,7 +523,10 @@ struct Solver {
       MXM_HIP(move_state<false>(pieces, q.p, til.ref_of.data(), Kd, (size_t)NP * NC, h, device, stream));
     else
       MXM_HIP(move_state<false>(pieces, f.p, til.ref_of.data(), Kd, (size_t)NP * NC, h, device, stream));
-    if (limiter) clear_pending();  // nothing pending on a new state
+    if (limiter)
+      clear_pending();  // nothing pending on a new state
+    else
+      stale = true;
   }
   void download_state(double *h) {
     if (prec == MXM_PREC_FP64)
@@ -816,7 +832,7 @@ int mxm_dg_enable_limiter(void *h, int on, double eps) {
   return guarded([&] {
     Solver *s = as_solver(h);
     if (s->NC > kLimMaxNC) throw ArgError("limiter supports NC <= " + std::to_string(kLimMaxNC));
-    if (on && !s->limiter) s->clear_pending();  // between calls the stored state is what it is
+    if (on && !s->limiter && s->stale) s->clear_limiter();
     s->limiter = on != 0;
     s->eps = eps;
     return MXM_OK;
@@ -933,6 +949,7 @@ int mxm_dg_time_stage_kernel(void *h, double dt, int nsteps, double *avg_us) {
     MXM_HIP(hipEventElapsedTime(&ms, ev[0], ev[1]));
     for (auto &e : ev) (void)hipEventDestroy(e);
     *avg_us = (double)ms * 1e3 / (3.0 * nsteps);
+    if (restore.lim) s->clear_limiter();  // nothing is pending on what these steps stored
     return MXM_OK;
   });
 }
