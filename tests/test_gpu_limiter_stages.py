@@ -72,3 +72,44 @@ def test_a_stage_after_steps(name, precision, nsteps):
                 s.rk_stage(2, dt)
                 out.append(s.get_state())
         assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("precision", [M.PREC_FP64, M.PREC_FP32_MFMA])
+@pytest.mark.parametrize("name", list(CASES))
+def test_switching_leaves_nothing_pending(name, precision):
+    """Off and on again, with a new state or steps in between, gives what a
+    solver gives that is handed the same state with the limiter on."""
+    phys, P, n = CASES[name]
+    print(name, precision, flush=True)
+    L = (1.0, 0.8, 1.2)[:len(n)]
+    dt = 0.05 * min(L) / max(n) / (2 * P + 1)
+    for between in ("nothing", "state", "steps", "timing"):
+        out = []
+        for switch in (True, False):
+            with M.Solver(n, L, phys, P=P, precision=precision) as s:
+                q, q2 = (random_state(phys, s.num_elements, s.NP, np.random.default_rng(k), len(n))
+                         .astype(np.float32).astype(np.float64) for k in (5, 6))
+                s.set_state(q)
+                s.enable_cell_limiter(True, 0.1)
+                s.step_ssprk3(dt, 3)
+                if between == "state":
+                    if switch:
+                        s.enable_cell_limiter(False)
+                    s.set_state(q2)
+                elif between == "steps":
+                    s.enable_cell_limiter(False)
+                    s.step_ssprk3(dt, 2)
+                    if not switch:  # nothing can be pending on a state that is set
+                        s.enable_cell_limiter(True, 0.1)
+                        s.set_state(s.get_state())
+                elif between == "timing":
+                    s.time_stage_kernel(dt, 1) if switch else None
+                    s.set_state(q2)
+                elif switch:
+                    s.enable_cell_limiter(False)
+                s.enable_cell_limiter(True, 0.1)
+                s.step_ssprk3(dt, 2)
+                s.rk_stage(2, dt)
+                out.append(s.get_state())
+        assert np.isfinite(out[0]).all()
+        assert np.array_equal(out[0], out[1]), between
