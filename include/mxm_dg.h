@@ -138,7 +138,9 @@ typedef struct {
     double mfma_utilization;  /* mfma_tflops / 157.3 (MI355X dense FP32 matrix peak); 0 in FP64 */
 } mxm_throughput;
 
-/* MemoryReport, src/memory_report.mojo:36-130 (six categories, bytes). */
+/* MemoryReport, src/memory_report.mojo:36-130 (six categories, bytes).
+ * Device memory of the solver; the pinned buffers of the state transfers (at
+ * most 16 MiB kept for the whole process) belong to no solver. */
 typedef struct {
     long long rk_stage;
     long long dg_operators;

@@ -66,7 +66,8 @@ __global__ __launch_bounds__(256) void bj_limit_kernel(R *__restrict__ q, double
     int nb[NF];
     bj_neighbours<NF>(e, conn, nb);
     const double th = bj_theta_comp<NC, ALL, NF>(e, t - el * NCL, nb, mean, ext, eps2, 1.0);
-    if (th < 1.0) atomicMin(reinterpret_cast<unsigned long long *>(&sTh[el]), (unsigned long long)__double_as_longlong(th));
+    if (th < 1.0)
+      atomicMin(reinterpret_cast<unsigned long long *>(&sTh[el]), (unsigned long long)__double_as_longlong(th));
   }
   __syncthreads();
   for (int t = tid; t < elems * NCL * 2; t += 256)

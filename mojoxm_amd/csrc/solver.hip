@@ -92,11 +92,11 @@ struct Solver {
   static constexpr int kGraphSteps = 32;
   // Calls of up to kDirectSteps steps launch their kernels on the stream: a
   // graph launch costs more than the launches it replaces (16^2 Alfven wave,
-  // one step per call: 22.7 -> 18.8 us per step; from 3 steps on the graph is
+  // one step per call: 22.7 -> 18.3 us per step; from 3 steps on the graph is
   // faster, 17.0).  So does the first call of up to kFirstSteps steps with a
   // new dt, as in a loop that clamps to its frames or follows the CFL speed:
-  // capturing and uploading a graph to use it once took 44 us for one step
-  // and 29 per step for three, the launches take 18.7.
+  // capturing and uploading a graph to use it once took 43.7 us for one
+  // step and 29 per step for three, the launches take 18.2.
   static constexpr int kDirectSteps = 2, kFirstSteps = 8;
   double last_dt = 0.0;  // of the last call that launched directly
   StepGraph gfull;
@@ -169,7 +169,8 @@ struct Solver {
   bool stale = true;
   // nothing pending on any stage buffer
   void clear_pending() {
-    MXM_HIP(launch_fill(reinterpret_cast<double *>(lext.p), (long long)(lext.n / sizeof(double)), no_extrema(), stream));
+    MXM_HIP(launch_fill(reinterpret_cast<double *>(lext.p), (long long)(lext.n / sizeof(double)), no_extrema(),
+                        stream));
   }
   void clear_limiter() {
     clear_pending();
@@ -913,8 +914,8 @@ int mxm_dg_memory_report(void *h, mxm_memory_report *o) {
     o->rk_stage = (long long)s->state_bytes();
     o->dg_operators = (long long)(s->Dt.bytes() + s->Lt.bytes() + s->Aop.bytes() + s->w.bytes() + s->fmap.bytes());
     o->limiter = (long long)(s->lmean.bytes() + s->ltheta.bytes() + s->lext.bytes());
-    o->mesh_connectivity = (long long)(s->conn.bytes() + s->geom.bytes() + s->geomf.bytes() + s->tile_type.bytes() + s->jobs.bytes() + s->ipr.bytes() +
-                                       s->tile_count.bytes());
+    o->mesh_connectivity = (long long)(s->conn.bytes() + s->geom.bytes() + s->geomf.bytes() + s->tile_type.bytes() +
+                                       s->jobs.bytes() + s->ipr.bytes() + s->tile_count.bytes());
     o->halo_device = 0;
     o->halo_pinned = 0;
     return MXM_OK;
