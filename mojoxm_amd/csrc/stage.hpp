@@ -1078,10 +1078,10 @@ dg_stage_kernel(StageArgs<R> A) {
   // sum_i w_i q_i per (element, component) in node order, FP64, from the
   // stored values: what a separate pass over q_out would compute
   if constexpr (LIM) {
-    // 35 and 56 nodes are not read all at once: Maxwell's FP64 kernel at P = 5
-    // held 132 VGPRs for that, 3 waves per SIMD where its LDS lets 4 run (15^3
-    // limited, us per stage: 242.7, 116 VGPRs 218.3)
-    constexpr int kUnroll = NP > 20 ? 8 : NP;
+    // FP64: 56 nodes are not read all at once.  Maxwell's kernel held 132 VGPRs
+    // for that, 3 waves per SIMD where its LDS lets 4 run (15^3 limited, us per
+    // stage: 242.7, in two halves 217.5); smaller elements and FP32 lose by it
+    constexpr int kUnroll = !kMFMA && NP == 56 ? 28 : NP;
     for (int p = tid; p < nE * NC; p += S::BLOCK) {
       const int el = p / NC, c = p - el * NC;
       double sm = 0.0;
